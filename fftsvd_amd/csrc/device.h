@@ -37,23 +37,18 @@ struct GemmDesc {
 };
 
 // Pivoted-MGS basis problem: A (rows x cols, column-major, column j at
-// a_off + j*rows, modified in place) -> rank and the first `rank`
+// a_off + j*lda, lda even and a_off even so that columns start 16-byte
+// aligned; modified in place) -> rank (rank_slot) and the first `rank`
 // orthonormal pivot columns at q_off (column k at q_off + k*rows).
-// seg lanes of a wave share one column; the problem's columns occupy the
-// update grid's waves wave0.. and its squared column norms sit at
-// ss_off.. (filled by the host scheduler).
+// seg, nb, ws_off are set by the host scheduler (run_mgs).
 struct MgsDesc {
-   int rows, cols;
+   int rows, cols, lda;
    long long a_off;
    long long q_off;
    int rank_slot;
-   int seg, wave0, ss_off, pid;   // pid: index of the problem's MgsState
-};
-
-// Per-problem progress of the stepwise MGS.
-struct MgsState {
-   double fro;
-   int rank, done;
+   int seg;             // register kernel: lanes per column pair
+   int nb;              // blocked kernel: steps per block
+   long long ws_off;    // blocked kernel: its arrays in the global scratch (when not in LDS)
 };
 
 // Near-field leaf: rows q0..q0+p-1 (tree-order points), m columns listed at
