@@ -12,7 +12,15 @@
 
 namespace fsvd {
 
-// A device buffer that frees itself.
+// Device memory for the buffers below (devmem.cpp): blocks given back are
+// kept (bounded) and taken again, so a block must be idle when it is given
+// back; dev_built tells that a problem has been built.
+void* dev_take(size_t bytes);
+void dev_give(void* p);
+void dev_built();
+
+// A device buffer that frees itself.  No work that uses it may be in flight
+// when it is destroyed or allocated anew.
 template <typename T>
 struct DBuf {
    T* p = nullptr;
@@ -36,14 +44,14 @@ struct DBuf {
    }
    ~DBuf() { reset(); }
    void reset() {
-      if (p) (void)hipFree(p);
+      if (p) dev_give(p);
       p = nullptr;
       n = 0;
    }
    void alloc(size_t count) {
       reset();
       n = count;
-      if (count) FSVD_CHECK(hipMalloc(&p, sizeof(T) * count));
+      if (count) p = (T*)dev_take(sizeof(T) * count);
    }
    void upload(const T* h, size_t count, hipStream_t s) {
       alloc(count);

@@ -97,6 +97,10 @@ static VT* basis_vec(Problem& pr, int j);
 static void reserve_solver_memory(Problem& pr, bool want32);
 
 Problem::~Problem() {
+   // every buffer idle before it is given back
+   if (stream) (void)hipStreamSynchronize(stream);
+   for (int k = 0; k < MAX_AUX; k++)
+      if (aux[k]) (void)hipStreamSynchronize(aux[k]);
    regions.clear();
    basis.clear();
    basis32.clear();
@@ -531,6 +535,7 @@ std::unique_ptr<Problem> build_problem(const SurfaceSpec& spec) {
    FSVD_CHECK(hipHostMalloc((void**)&pr.h_pinned, sizeof(double) * 2048));
    reserve_solver_memory(pr, spec.want32);
    FSVD_CHECK(hipStreamSynchronize(s));
+   dev_built();
    pr.setup_ms = now_ms() - t0;
    setup_event("problem end");
    return prp;
@@ -620,6 +625,7 @@ std::unique_ptr<Problem> build_qual_problem(const QualSpec& spec) {
    FSVD_CHECK(hipHostMalloc((void**)&pr.h_pinned, sizeof(double) * 2048));
    reserve_solver_memory(pr, spec.want32);
    FSVD_CHECK(hipStreamSynchronize(s));
+   dev_built();
    pr.setup_ms = now_ms() - t0;
    return prp;
 }
@@ -840,6 +846,7 @@ static const VT* const* basis_ptrs(Problem& pr, int m) {
       const int cap = ((m + 63) / 64) * 64;
       std::vector<const VT*> p(cap);
       for (int j = 0; j < cap; j++) p[j] = basis_vec<VT>(pr, j);
+      FSVD_CHECK(hipStreamSynchronize(pr.stream));   // steps in flight read the old array
       if constexpr (f64)
          pr.d_basis_ptr.upload(p, pr.stream);
       else
@@ -1159,6 +1166,7 @@ static const VT* const* col_basis_ptrs(Problem& pr, GmCol& g, int m) {
       const int cap = ((m + 63) / 64) * 64;
       std::vector<const VT*> p(cap);
       for (int j = 0; j < cap; j++) p[j] = col_basis<VT>(pr, g, j);
+      FSVD_CHECK(hipStreamSynchronize(pr.stream));   // steps in flight read the old array
       if constexpr (f64)
          g.ptr64.upload(p, pr.stream);
       else
@@ -1495,6 +1503,7 @@ void problem_potentials(Problem& pr, const double* sol, double* phi_out, bool us
       dsf.upload(self, s);
       dc.upload(coef, s);
       launch_potentials(nq, pr.ntotal, pr.regions[0].d_panels.p, dp.p, dc.p, dsf.p, pr.d_qpos.p, dphi.p, s);
+      FSVD_CHECK(hipStreamSynchronize(s));
    }
    for (Region& R : pr.regions) {
       if (pr.qual || !R.m3 || !use_m3) continue;
