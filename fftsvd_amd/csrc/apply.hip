@@ -6,8 +6,8 @@
 // Storage precision T is float (mixed mode) or double (FP64 mode); vectors
 // enter and leave in FP64.  The forward apply is five launches per tree
 // (k_project, k_source, k_translate, k_target, k_leaf; each covers every
-// level).  The transposed operator (k_farT_*, k_far_translate, k_nearT)
-// runs level by level with the roles of the two sides swapped.
+// level).  The transposed operator runs the same stages with the roles of the
+// two sides swapped and one input vector, and k_leaf_t for its output.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -192,29 +192,6 @@ struct FarSizes {
    static constexpr int N = 2 * n - 1, H = N / 2 + 1, PAD = N * N * H, GP3 = n * n * n;
 };
 
-// Translation: S_d[b] = sum_e T[toff_e][b] * G[src_e][b].  Blocks
-// (target cube, slice of gridDim.y over the bins), threads over bins; each
-// bin's sum is the same whatever the slicing.
-template <typename T>
-__global__ void __launch_bounds__(256) k_far_translate(const TgtDesc* __restrict__ tgt,
-                                                       const int* __restrict__ int_src,
-                                                       const int* __restrict__ int_toff,
-                                                       const typename Cplx<T>::type* __restrict__ Tspec,
-                                                       const typename Cplx<T>::type* __restrict__ spec,
-                                                       typename Cplx<T>::type* __restrict__ acc, int pad) {
-   const TgtDesc d = tgt[blockIdx.x];
-   for (int b = threadIdx.x + (int)(blockIdx.y * blockDim.x); b < pad; b += (int)(blockDim.x * gridDim.y)) {
-      T re = 0, im = 0;
-      for (int e = 0; e < d.nint; e++) {
-         auto t = Tspec[(long long)int_toff[d.int_off + e] * pad + b];
-         auto s = spec[(long long)int_src[d.int_off + e] * pad + b];
-         re += t.x * s.x - t.y * s.y;
-         im += t.x * s.y + t.y * s.x;
-      }
-      acc[(long long)d.spec_slot * pad + b] = {re, im};
-   }
-}
-
 // ---------------------------------------------------------------------------
 // Forward apply, one launch per stage over all levels of a tree:
 //   k_project    chunk of a source cube's panels: partial VT.xs, VT.xd
@@ -276,11 +253,11 @@ __device__ __forceinline__ T stream_rows(const T* __restrict__ colp, int E, int 
 }
 
 // Projection: one chunk of a source cube's panels per wavefront (four per
-// block), tpart[out_off + e] = sum_i VT[e, i] xs[i] and
+// block), tpart[out_off + e] = sum_i VT[e, i] xs[i] and, with two layers (NL),
 // tpart[out_off + r + e] = sum_i VT[e, i] xd[i] over the chunk's columns.
 // Lane (g, e) owns row e and the columns g, g + G, ... (G = 64 / rows of the
 // row chunk); the G partial sums of a row are added in group order.
-template <typename T, bool NT>
+template <typename T, bool NT, int NL>
 __global__ void __launch_bounds__(256) k_project(const ProjChunk* __restrict__ chunks, int nchunk,
                                                  const T* __restrict__ VTc, const double* __restrict__ xs,
                                                  const double* __restrict__ xd, T* __restrict__ tpart, int wave_lds,
@@ -290,13 +267,13 @@ __global__ void __launch_bounds__(256) k_project(const ProjChunk* __restrict__ c
    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, ci = cb.b * 4 + wave;
    if (ci >= nchunk) return;
    xs += cb.c * cs_x;
-   xd += cb.c * cs_x;
+   if (NL == 2) xd += cb.c * cs_x;
    tpart += cb.c * cs_tpart;
    const WaveGroup gr{lane};
    const ProjChunk c = chunks[ci];
    const int m = c.ncol, E = c.r;
-   T* part = (T*)(smem + (size_t)wave * wave_lds);   // 2*64
-   T* xl = part + 128;                                // 2*m
+   T* part = (T*)(smem + (size_t)wave * wave_lds);   // NL*64
+   T* xl = part + NL * 64;                            // NL*m
    // x staged four columns per lane at a time, loads before stores
    for (int i0 = lane; i0 < m; i0 += 256) {
       double a[4], b[4];
@@ -304,14 +281,14 @@ __global__ void __launch_bounds__(256) k_project(const ProjChunk* __restrict__ c
       for (int u = 0; u < 4; u++) {
          const int i = i0 + 64 * u;
          a[u] = i < m ? xs[c.p0 + i] : 0.0;
-         b[u] = i < m ? xd[c.p0 + i] : 0.0;
+         b[u] = NL == 2 && i < m ? xd[c.p0 + i] : 0.0;
       }
 #pragma unroll
       for (int u = 0; u < 4; u++) {
          const int i = i0 + 64 * u;
          if (i < m) {
             xl[i] = (T)a[u];
-            xl[m + i] = (T)b[u];
+            if (NL == 2) xl[m + i] = (T)b[u];
          }
       }
    }
@@ -334,9 +311,9 @@ __global__ void __launch_bounds__(256) k_project(const ProjChunk* __restrict__ c
 #pragma unroll
             for (int u = 0; u < 8; u += 2) {
                s0 += v[u] * xl[i + u * G];
-               d0 += v[u] * xl[m + i + u * G];
+               if (NL == 2) d0 += v[u] * xl[m + i + u * G];
                s1 += v[u + 1] * xl[i + (u + 1) * G];
-               d1 += v[u + 1] * xl[m + i + (u + 1) * G];
+               if (NL == 2) d1 += v[u + 1] * xl[m + i + (u + 1) * G];
             }
          }
          if (i < m) {
@@ -349,23 +326,23 @@ __global__ void __launch_bounds__(256) k_project(const ProjChunk* __restrict__ c
             for (int u = 0; u < 7; u++)
                if (i + u * G < m) {
                   s0 += v[u] * xl[i + u * G];
-                  d0 += v[u] * xl[m + i + u * G];
+                  if (NL == 2) d0 += v[u] * xl[m + i + u * G];
                }
          }
          as = s0 + s1;
          ad = d0 + d1;
       }
       part[lane] = as;
-      part[64 + lane] = ad;
+      if (NL == 2) part[64 + lane] = ad;
       gr.sync();
       if (lane < Ec) {
          T ss = 0, sd = 0;
          for (int gg = 0; gg < G; gg++) {
             ss += part[gg * Ec + lane];
-            sd += part[64 + gg * Ec + lane];
+            if (NL == 2) sd += part[64 + gg * Ec + lane];
          }
          tpart[c.out_off + e0 + lane] = ss;
-         tpart[c.out_off + E + e0 + lane] = sd;
+         if (NL == 2) tpart[c.out_off + E + e0 + lane] = sd;
       }
       gr.sync();
    }
@@ -482,7 +459,7 @@ __global__ void __launch_bounds__(256) k_project_mc(const ProjChunk* __restrict_
    }
 }
 
-template <int n, typename T, bool NT, typename G>
+template <int n, typename T, bool NT, int NL, typename G>
 __device__ void source_body(const SrcPlan& d, const T* __restrict__ tpart, const T* __restrict__ PV,
                             typename Cplx<T>::type* __restrict__ spec, unsigned char* smem, const G& gr) {
    using C2 = typename Cplx<T>::type;
@@ -493,25 +470,25 @@ __device__ void source_body(const SrcPlan& d, const T* __restrict__ tpart, const
    T* sn = cs + N;               // N
    T* g = sn + N;                // GP3
    T* part = g + GP3;            // partial grid values (block groups)
-   const int tid = gr.tid, nt = gr.nt, r = d.r;
-   T* t = part + (nt > GP3 ? nt : 0);   // 2r: ts then td
+   const int tid = gr.tid, nt = gr.nt, R2 = NL * d.r;
+   T* t = part + (nt > GP3 ? nt : 0);   // NL*r: ts then td
    twiddle_table<T, N>(cs, sn, gr);
    // sum of the chunk partials in chunk order, eight loads in flight
-   for (int k = tid; k < 2 * r; k += nt) {
+   for (int k = tid; k < R2; k += nt) {
       const T* pp = tpart + d.part_off + k;
       T a = 0;
       int j = 0;
       for (; j + 7 < d.nchunk; j += 8) {
          T v[8];
 #pragma unroll
-         for (int u = 0; u < 8; u++) v[u] = pp[(long long)(j + u) * 2 * r];
+         for (int u = 0; u < 8; u++) v[u] = pp[(long long)(j + u) * R2];
 #pragma unroll
          for (int u = 0; u < 8; u++) a += v[u];
       }
       if (j < d.nchunk) {
          T v[7];
 #pragma unroll
-         for (int u = 0; u < 7; u++) v[u] = j + u < d.nchunk ? pp[(long long)(j + u) * 2 * r] : (T)0;
+         for (int u = 0; u < 7; u++) v[u] = j + u < d.nchunk ? pp[(long long)(j + u) * R2] : (T)0;
 #pragma unroll
          for (int u = 0; u < 7; u++)
             if (j + u < d.nchunk) a += v[u];
@@ -519,10 +496,9 @@ __device__ void source_body(const SrcPlan& d, const T* __restrict__ tpart, const
       t[k] = a;
    }
    gr.sync();
-   // g = PV t over the 2r rows (PVs then PVd, k-major): thread (kg, q) sums
+   // g = PV t over the rows (PVs then PVd, k-major): thread (kg, q) sums
    // the rows k = kg, kg + KG, ... so every thread streams PV
    const T* pv = PV + d.pv_off;
-   const int R2 = 2 * r;
    const int KG = nt >= GP3 ? nt / GP3 : 1, QW = nt / KG;
    for (int q0 = 0; q0 < GP3; q0 += QW) {
       const int kg = tid / QW, q = q0 + tid - kg * QW;
@@ -586,7 +562,7 @@ __host__ __device__ constexpr size_t source_cube_lds(int n, int maxr, int nt) {
 // block, each wave in its own LDS slice of wave_lds bytes.  The small cubes
 // run while the large ones finish.
 constexpr int CUBE_NT = 512;
-template <typename T, bool NT>
+template <typename T, bool NT, int NL>
 __global__ void __launch_bounds__(CUBE_NT) k_source(const SrcPlan* __restrict__ src, int nbig, int nsrc,
                                                     const T* __restrict__ tpart, const T* __restrict__ PV,
                                                     typename Cplx<T>::type* __restrict__ spec, int wave_lds, int nb,
@@ -600,12 +576,12 @@ __global__ void __launch_bounds__(CUBE_NT) k_source(const SrcPlan* __restrict__ 
       const SrcPlan d = src[cb.b];
       const BlockGroup gr = block_group();
       switch (d.n) {
-         case 3: source_body<3, T, NT>(d, tpart, PV, spec, smem, gr); break;
-         case 5: source_body<5, T, NT>(d, tpart, PV, spec, smem, gr); break;
-         case 6: source_body<6, T, NT>(d, tpart, PV, spec, smem, gr); break;
-         case 7: source_body<7, T, NT>(d, tpart, PV, spec, smem, gr); break;
-         case 8: source_body<8, T, NT>(d, tpart, PV, spec, smem, gr); break;
-         case 9: source_body<9, T, NT>(d, tpart, PV, spec, smem, gr); break;
+         case 3: source_body<3, T, NT, NL>(d, tpart, PV, spec, smem, gr); break;
+         case 5: source_body<5, T, NT, NL>(d, tpart, PV, spec, smem, gr); break;
+         case 6: source_body<6, T, NT, NL>(d, tpart, PV, spec, smem, gr); break;
+         case 7: source_body<7, T, NT, NL>(d, tpart, PV, spec, smem, gr); break;
+         case 8: source_body<8, T, NT, NL>(d, tpart, PV, spec, smem, gr); break;
+         case 9: source_body<9, T, NT, NL>(d, tpart, PV, spec, smem, gr); break;
          default: break;
       }
       return;
@@ -613,7 +589,7 @@ __global__ void __launch_bounds__(CUBE_NT) k_source(const SrcPlan* __restrict__ 
    const int wave = threadIdx.x >> 6, i = nbig + (cb.b - nbig) * (CUBE_NT / 64) + wave;
    if (i >= nsrc) return;
    const SrcPlan d = src[i];
-   source_body<4, T, NT>(d, tpart, PV, spec, smem + (size_t)wave * wave_lds, WaveGroup{(int)(threadIdx.x & 63)});
+   source_body<4, T, NT, NL>(d, tpart, PV, spec, smem + (size_t)wave * wave_lds, WaveGroup{(int)(threadIdx.x & 63)});
 }
 
 // FP64 translation by tiles: a block owns BC frequency bins (one TR_ROW-byte
@@ -1754,170 +1730,161 @@ __global__ void __launch_bounds__(256) k_leaf_mc(const LeafDesc* __restrict__ le
    }
 }
 
-__global__ void k_zero(double* __restrict__ a, long long n) {
-   for (long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x; i < n; i += (long long)gridDim.x * blockDim.x)
-      a[i] = 0.0;
-}
-
 // ---------------------------------------------------------------------------
-// Transposed operator of one layer (reference Tree_multiply_transpose,
-// Tree.c:769-832).  Points side forward: u = U^T x, h = UTI^T u, DFT.  Any
-// block size gives the same results (one wave per row of U^T, one thread
-// per grid value); the coarse levels, with few large cubes, run 16 waves
-// per cube.
-template <int n, typename T>
-__global__ void __launch_bounds__(1024) k_farT_source(const TgtDesc* __restrict__ tgt, const T* __restrict__ UT,
-                                                     const T* __restrict__ UTI, const double* __restrict__ x,
-                                                     typename Cplx<T>::type* __restrict__ spec, int maxr) {
-   using C2 = typename Cplx<T>::type;
-   constexpr int N = FarSizes<n>::N, H = FarSizes<n>::H, PAD = FarSizes<n>::PAD, GP3 = FarSizes<n>::GP3;
-   extern __shared__ __align__(16) unsigned char smem[];
-   C2* A = (C2*)smem;
-   C2* B = A + n * n * H;
-   T* cs = (T*)(B + n * N * H);
-   T* sn = cs + N;
-   T* g = sn + N;
-   T* u = g + GP3;
-   const TgtDesc d = tgt[blockIdx.x];
-   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, nw = blockDim.x >> 6;
-   twiddle_table<T, N>(cs, sn);
-   const T* ut = UT + d.u_off;
-   for (int k = wave; k < d.r; k += nw) {
-      const T* row = ut + (long long)k * d.nq;
-      T a = 0;
-      for (int i = lane; i < d.nq; i += 64) a += row[i] * (T)x[d.q0 + i];
-      a = wave_sum(a);
-      if (lane == 0) u[k] = a;
-   }
-   __syncthreads();
-   const T* uti = UTI + d.uti_off;
-   for (int q = tid; q < GP3; q += blockDim.x) {
-      T a = 0;
-      for (int k = 0; k < d.r; k++) a += uti[(long long)k * GP3 + q] * u[k];
-      g[q] = a;
-   }
-   __syncthreads();
-   grid_forward<n, T>(g, A, B, spec + (long long)d.spec_slot * PAD, cs, sn);
-}
-
-// Panels side backward: h = IDFT, w = PV_layer^T h, y[panels] += VT^T w.
-// The cube's panels are cut into gridDim.y contiguous chunks, one block
-// each (every block forms the same h and w; each output is written by one
-// block with the arithmetic of the unsplit kernel), so that the coarse
-// levels' few large cubes occupy more than one CU each.
-template <int n, typename T>
-__global__ void __launch_bounds__(256) k_farT_target(const SrcDesc* __restrict__ src, const T* __restrict__ VT,
-                                                     const T* __restrict__ PV,
-                                                     const typename Cplx<T>::type* __restrict__ acc, int layer,
-                                                     double* __restrict__ yfar, double* __restrict__ yfar2,
-                                                     int maxr) {
-   using C2 = typename Cplx<T>::type;
-   constexpr int N = FarSizes<n>::N, H = FarSizes<n>::H, PAD = FarSizes<n>::PAD, GP3 = FarSizes<n>::GP3;
-   extern __shared__ __align__(16) unsigned char smem[];
-   C2* S = (C2*)smem;
-   C2* C1 = S + PAD;
-   C2* Cc = C1 + n * N * H;
-   T* cs = (T*)(Cc + n * n * H);
-   T* sn = cs + N;
-   T* h = sn + N;
-   T* w = h + GP3;
-   const SrcDesc d = src[blockIdx.x];
-   const int chunk = (d.np + (int)gridDim.y - 1) / (int)gridDim.y;
-   const int i0 = (int)blockIdx.y * chunk, i1 = i0 + chunk < d.np ? i0 + chunk : d.np;
-   if (i0 >= i1) return;   // uniform over the block
-   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, nw = blockDim.x >> 6;
-   twiddle_table<T, N>(cs, sn);
-   for (int b = tid; b < PAD; b += blockDim.x) S[b] = acc[(long long)d.spec_slot * PAD + b];
-   __syncthreads();
-   grid_backward<n, T>(S, C1, Cc, h, cs, sn);
-   __syncthreads();
-   // yfar2 set: both layers from the one inverse transform (single layer
-   // into yfar, double layer into yfar2), each summed as alone
-   const int nl = yfar2 ? 2 : 1;
-   for (int li = 0; li < nl; li++) {
-      const T* pv = PV + d.pv_off + ((yfar2 ? li : layer) ? (long long)d.r * GP3 : 0);
-      for (int k = wave; k < d.r; k += nw) {
-         const T* row = pv + (long long)k * GP3;
-         T a = 0;
-         for (int q = lane; q < GP3; q += 64) a += row[q] * h[q];
-         a = wave_sum(a);
-         if (lane == 0) w[li * d.r + k] = a;
-      }
-   }
-   __syncthreads();
-   const T* vt = VT + d.vt_off;
-   for (int li = 0; li < nl; li++) {
-      double* out = li ? yfar2 : yfar;
-      for (int i = i0 + tid; i < i1; i += blockDim.x) {
-         T a = 0;
-         for (int k = 0; k < d.r; k++) a += vt[(long long)k * d.np + i] * w[li * d.r + k];
-         out[d.p0 + i] += (double)a;
-      }
-   }
-}
-
-// Near field transposed: y[cols] += D_layer^T x[rows] (global atomics; columns
-// are shared between neighbouring leaves).
-// With y2: both layers (single into y, double into y2) from one pass over
-// the block.
+// Output of the transposed apply (reference Tree_multiply_transpose,
+// Tree.c:769-832), one block per leaf (up to LT_SLAB of its panels): for its panels i
+//   ys[i] = sum of the single-layer column i of every near-field block that
+//           holds it, times x, plus sum_k VT[k, i] ws[k] over the leaf's source
+//           cubes; yd likewise for the double layer.
+// Gathered per leaf, so each near-field entry is read once and no output is
+// shared between blocks (one scatter per block with FP64 atomics took 87 us a
+// tree at 31 000 panels, beside ~60 per-level launches for the far field).
+// Bound by latency: short gathers (32 rows per neighbour block, 20-60 columns),
+// 39 us a launch at 31 000 panels with 7 waves per SIMD.  Transposed product of
+// both trees, host to host: 31 000 panels 1.22 to 0.28 ms FP32, 1.49 to 0.39
+// FP64; 100 000 panels 2.38 to 0.67 and 2.89 to 1.03.  Near field: the rows of all blocks are listed in
+// LDS (TILE at a time: entry offset, column stride, x), lanes take rows, waves
+// four columns each with both layers of a column in flight; FP64 sums.  Far
+// field: 16 lanes per panel over the rows of its panel-major basis, summed in
+// T per source cube and in FP64 over the cubes.
+constexpr int LT_TILE = 512;
 template <typename T>
-__global__ void __launch_bounds__(256) k_nearT(const LeafDesc* __restrict__ leaves, const int* __restrict__ dcol,
-                                               const T* __restrict__ D, const double* __restrict__ x, int layer,
-                                               double* __restrict__ y, double* __restrict__ y2) {
-   const LeafDesc L = leaves[blockIdx.x];
-   const T* blk = D + L.d_off + ((layer && !y2) ? L.p : 0);
-   for (int c = threadIdx.x; c < L.m; c += blockDim.x) {
-      const T* colp = blk + (long long)c * 2 * L.p;
-      double a = 0.0;
-      for (int r = 0; r < L.p; r++) a += (double)colp[r] * x[L.q0 + r];
-      atomicAdd(&y[dcol[L.col_off + c]], a);
-      if (y2) {
-         double b = 0.0;
-         for (int r = 0; r < L.p; r++) b += (double)colp[L.p + r] * x[L.q0 + r];
-         atomicAdd(&y2[dcol[L.col_off + c]], b);
+__global__ void __launch_bounds__(256, sizeof(T) == 4 ? 7 : 5) k_leaf_t(const LeafT* __restrict__ leaves, const NearT* __restrict__ nbr,
+                                                const T* __restrict__ D, const double* __restrict__ x,
+                                                const LeafU* __restrict__ ublk, const T* __restrict__ VTc,
+                                                const T* __restrict__ w, double* __restrict__ ys,
+                                                double* __restrict__ yd) {
+   extern __shared__ __align__(16) unsigned char smem[];
+   __shared__ double xr[LT_TILE];
+   __shared__ long long base[LT_TILE];
+   __shared__ int st[LT_TILE];
+   constexpr int CW = 4, RU = 2;
+   const LeafT L = leaves[blockIdx.x];   // in launch order; np = 0: idle
+   if (L.np == 0) return;
+   double* res = (double*)smem;   // near field: np single-layer, then np double-layer sums
+   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, grp = tid >> 4, gl = tid & 15;
+   for (int cb = 0; cb < L.np; cb += 4 * CW) {
+      const int c0 = cb + CW * wave;
+      double as[CW], ad[CW];
+#pragma unroll
+      for (int c = 0; c < CW; c++) as[c] = ad[c] = 0.0;
+      for (int t0 = 0; t0 < L.rows; t0 += LT_TILE) {
+         const int tn = min(LT_TILE, L.rows - t0);
+         // one tile holds the rows of most leaves: listed once
+         if (cb == 0 || L.rows > LT_TILE) {
+            __syncthreads();
+            for (int j = grp; j < L.nn; j += 16) {
+               const NearT e = nbr[L.nb0 + j];
+               for (int r = gl; r < e.p; r += 16) {
+                  const int i = e.row0 + r - t0;
+                  if (i >= 0 && i < tn) {
+                     xr[i] = x[e.q0 + r];
+                     base[i] = e.d_off + r;
+                     st[i] = 2 * e.p;
+                  }
+               }
+            }
+            __syncthreads();
+         }
+         if (c0 < L.np)
+            for (int i0 = lane; i0 < tn; i0 += 64 * RU) {
+               // RU rows per lane in flight; a row past the last repeats it
+               // with x = 0, a column past the last repeats it (sum unused)
+               T vs[RU][CW], vd[RU][CW];
+               double xi[RU];
+#pragma unroll
+               for (int q = 0; q < RU; q++) {
+                  const int i = min(i0 + 64 * q, tn - 1);
+                  xi[q] = i0 + 64 * q < tn ? xr[i] : 0.0;
+                  const int sc = st[i];
+                  const T* p = D + base[i];
+#pragma unroll
+                  for (int c = 0; c < CW; c++) {
+                     const T* pc = p + (long long)min(c0 + c, L.np - 1) * sc;
+                     if (ys) vs[q][c] = pc[0];
+                     if (yd) vd[q][c] = pc[sc >> 1];
+                  }
+               }
+#pragma unroll
+               for (int q = 0; q < RU; q++)
+#pragma unroll
+                  for (int c = 0; c < CW; c++) {
+                     if (ys) as[c] = fma((double)vs[q][c], xi[q], as[c]);
+                     if (yd) ad[c] = fma((double)vd[q][c], xi[q], ad[c]);
+                  }
+            }
+      }
+#pragma unroll
+      for (int c = 0; c < CW; c++) {
+         if (c0 + c < L.np) {   // uniform over the wave
+            const double s = ys ? wave_sum(as[c]) : 0.0, d = yd ? wave_sum(ad[c]) : 0.0;
+            if (lane == 0) {
+               res[c0 + c] = s;
+               res[L.np + c0 + c] = d;
+            }
+         }
+      }
+   }
+   __syncthreads();
+   for (int i0 = 0; i0 < L.np; i0 += 16) {
+      const int i = i0 + grp, ic = min(i, L.np - 1);
+      double as = 0.0, ad = 0.0;
+      // four source cubes at a time, their loads in flight together
+      for (int u0 = 0; u0 < L.nu; u0 += 4) {
+         LeafU b[4];
+#pragma unroll
+         for (int u = 0; u < 4; u++) b[u] = ublk[L.u0 + min(u0 + u, L.nu - 1)];
+         T a[4] = {0, 0, 0, 0}, d[4] = {0, 0, 0, 0};
+         int rmax = 0;
+#pragma unroll
+         for (int u = 0; u < 4; u++) {
+            if (u0 + u >= L.nu) b[u].r = 0;
+            rmax = max(rmax, b[u].r);
+         }
+         for (int k0 = gl; k0 < rmax; k0 += 32) {
+            T vv[4][2], sv[4][2], dv[4][2];
+#pragma unroll
+            for (int u = 0; u < 4; u++)
+#pragma unroll
+               for (int q = 0; q < 2; q++) {
+                  // clamped index, selected sums: no branch around the loads
+                  const int k = k0 + 16 * q < b[u].r ? k0 + 16 * q : 0;
+                  vv[u][q] = VTc[b[u].u_off + (long long)ic * b[u].ld + k];
+                  if (ys) sv[u][q] = w[b[u].w_off + k];
+                  if (yd) dv[u][q] = w[b[u].w_off + b[u].ld + k];
+               }
+#pragma unroll
+            for (int u = 0; u < 4; u++)
+#pragma unroll
+               for (int q = 0; q < 2; q++) {
+                  const T m = k0 + 16 * q < b[u].r ? vv[u][q] : (T)0;
+                  if (ys) a[u] += m * sv[u][q];
+                  if (yd) d[u] += m * dv[u][q];
+               }
+         }
+#pragma unroll
+         for (int u = 0; u < 4; u++) {
+            as += (double)a[u];
+            ad += (double)d[u];
+         }
+      }
+#pragma unroll
+      for (int o = 8; o > 0; o >>= 1) {
+         as += __shfl_xor(as, o, 64);
+         ad += __shfl_xor(ad, o, 64);
+      }
+      if (gl == 0 && i < L.np) {
+         if (ys) ys[L.p0 + i] = res[i] + as;
+         if (yd) yd[L.p0 + i] = res[L.np + i] + ad;
       }
    }
 }
 
 // ---------------------------------------------------------------------------
 // Explicit instantiations and launchers
-template <typename T>
-size_t far_source_lds(int n, int maxr) {
-   int N = 2 * n - 1, H = N / 2 + 1;
-   return sizeof(typename Cplx<T>::type) * (size_t)(n * n * H + n * N * H) +
-          sizeof(T) * (size_t)(2 * N + n * n * n + 256 + 2 * maxr) + 64;
-}
-template <typename T>
-size_t far_target_lds(int n, int maxr) {
-   int N = 2 * n - 1, H = N / 2 + 1;
-   return sizeof(typename Cplx<T>::type) * (size_t)(N * N * H + n * N * H + n * n * H) + sizeof(T) * (size_t)(2 * N + n * n * n + maxr) + 64;
-}
-
-#define FSVD_DISPATCH_N(n, CALL) \
-   switch (n) {                  \
-      case 3: CALL(3); break;    \
-      case 4: CALL(4); break;    \
-      case 5: CALL(5); break;    \
-      case 6: CALL(6); break;    \
-      case 7: CALL(7); break;    \
-      case 8: CALL(8); break;    \
-      case 9: CALL(9); break;    \
-      default: throw std::runtime_error("unsupported grid size"); \
-   }
-
 // gfx950: 160 KiB of LDS per workgroup
 static void check_lds(size_t lds) {
    if (lds > 163840) throw std::runtime_error("LDS request above 160 KiB per workgroup");
-}
-
-template <typename T>
-void launch_far_translate(int nblk, const TgtDesc* tgt, const int* isrc, const int* itoff, const void* Tspec,
-                          const void* spec, void* acc, int pad, hipStream_t s) {
-   // one block per 256 bins of each cube (the coarse levels have few cubes)
-   const int slices = std::max(1, std::min(8, (pad + 255) / 256));
-   hipLaunchKernelGGL((k_far_translate<T>), dim3(nblk, slices), dim3(256), 0, s, tgt, isrc, itoff,
-                      (const typename Cplx<T>::type*)Tspec, (const typename Cplx<T>::type*)spec,
-                      (typename Cplx<T>::type*)acc, pad);
 }
 
 void launch_translate_pipe(int nblk, int mode, const int2* range, const int4* tasks, const TpTile* tiles,
@@ -1952,9 +1919,9 @@ void launch_apply_stage(int stage, const ApplyArgs& a, hipStream_t s) {
          const int wl = (int)((sizeof(T) * (size_t)(2 * a.proj_maxcols + 128) + 15) / 16 * 16);
          check_lds(4 * (size_t)wl);
          if (a.nchunk && a.ncol == 1) {
-            hipLaunchKernelGGL((k_project<T, true>), dim3((a.nchunk + 3) / 4), dim3(256), 4 * (size_t)wl, s,
-                               a.chunks, a.nchunk, (const T*)a.VTc, a.xs, a.xd, (T*)a.tpart, wl, 1, a.cs_x,
-                               a.cs_tpart);
+            auto kern = a.layers == 1 ? k_project<T, true, 1> : k_project<T, true, 2>;
+            hipLaunchKernelGGL(kern, dim3((a.nchunk + 3) / 4), dim3(256), 4 * (size_t)wl, s, a.chunks, a.nchunk,
+                               (const T*)a.VTc, a.xs, a.xd, (T*)a.tpart, wl, 1, a.cs_x, a.cs_tpart);
          } else if (a.nchunk) {
             constexpr int NC = proj_nc<T>();
             const int wlm = (int)((sizeof(T) * (size_t)NC * (2 * a.proj_maxcols + 128) + 15) / 16 * 16);
@@ -1979,14 +1946,16 @@ void launch_apply_stage(int stage, const ApplyArgs& a, hipStream_t s) {
          check_lds(lds);
          static std::once_flag attr;   // large n needs more than the default dynamic LDS
          std::call_once(attr, [] {
-            FSVD_CHECK(hipFuncSetAttribute((const void*)k_source<T, true>,
+            FSVD_CHECK(hipFuncSetAttribute((const void*)k_source<T, true, 2>,
                                            hipFuncAttributeMaxDynamicSharedMemorySize, 163840));
-            FSVD_CHECK(hipFuncSetAttribute((const void*)k_source<T, false>,
+            FSVD_CHECK(hipFuncSetAttribute((const void*)k_source<T, false, 2>,
+                                           hipFuncAttributeMaxDynamicSharedMemorySize, 163840));
+            FSVD_CHECK(hipFuncSetAttribute((const void*)k_source<T, true, 1>,
                                            hipFuncAttributeMaxDynamicSharedMemorySize, 163840));
          });
          const int nb = a.nsrc_big + (a.nsrc - a.nsrc_big + CUBE_NT / 64 - 1) / (CUBE_NT / 64);
          if (nb) {
-            auto kern = a.ncol == 1 ? k_source<T, true> : k_source<T, false>;
+            auto kern = a.layers == 1 ? k_source<T, true, 1> : (a.ncol == 1 ? k_source<T, true, 2> : k_source<T, false, 2>);
             hipLaunchKernelGGL(kern, dim3(col_grid(nb, a.ncol)), dim3(CUBE_NT), lds, s, a.src, a.nsrc_big, a.nsrc,
                                (const T*)a.tpart, (const T*)a.PV, (C2*)a.spec, wl, nb, a.ncol, a.cs_tpart,
                                a.cs_spec);
@@ -2091,6 +2060,13 @@ void launch_apply_stage(int stage, const ApplyArgs& a, hipStream_t s) {
          }
          break;
       }
+      case 5: {
+         const size_t lds = sizeof(double) * 2 * (size_t)std::max(a.maxnpT, 1);   // at most 16 LT_SLAB bytes
+         if (a.nleafT)
+            hipLaunchKernelGGL((k_leaf_t<T>), dim3(a.nleafT), dim3(256), lds, s, a.leavesT, a.nbrT, (const T*)a.D,
+                               a.xs, a.ublk, (const T*)a.VTc, (const T*)a.w, a.y, a.y2);
+         break;
+      }
       default: break;
    }
 }
@@ -2113,58 +2089,9 @@ void launch_transpose_batched(int n, const TransDesc* d, hipStream_t s) {
       hipLaunchKernelGGL((k_transpose_batched<T>), dim3(std::min(65535, n - b0)), dim3(256), 0, s, d + b0);
 }
 
-template <typename T>
-void launch_farT_source(int n, int nblk, const TgtDesc* tgt, const T* UT, const T* UTI, const double* x, void* spec,
-                        int maxr, hipStream_t s) {
-   size_t lds = far_source_lds<T>(n, maxr);
-   check_lds(lds);
-   const int threads = n >= 5 ? 1024 : 256;
-#define CALL(NN)                                                                                                    \
-   hipLaunchKernelGGL((k_farT_source<NN, T>), dim3(nblk), dim3(threads), lds, s, tgt, UT, UTI, x,                  \
-                      (typename Cplx<T>::type*)spec, maxr)
-   FSVD_DISPATCH_N(n, CALL)
-#undef CALL
-}
-
-template <typename T>
-void launch_farT_target(int n, int nblk, const SrcDesc* src, const T* VT, const T* PV, const void* acc, int layer,
-                        double* yfar, double* yfar2, int maxr, hipStream_t s) {
-   size_t lds = far_target_lds<T>(n, yfar2 ? 2 * maxr : maxr);
-   check_lds(lds);
-   // panel chunks per cube: the coarse levels (more grid points) have few,
-   // large cubes
-   const int split = n >= 6 ? 8 : (n == 5 ? 4 : 1);
-#define CALL(NN)                                                                                                    \
-   hipLaunchKernelGGL((k_farT_target<NN, T>), dim3(nblk, split), dim3(256), lds, s, src, VT, PV,                   \
-                      (const typename Cplx<T>::type*)acc, layer, yfar, yfar2, maxr)
-   FSVD_DISPATCH_N(n, CALL)
-#undef CALL
-}
-
-template <typename T>
-void launch_nearT(int nleaf, const LeafDesc* leaves, const int* dcol, const T* D, const double* x, int layer,
-                  double* y, double* y2, hipStream_t s) {
-   hipLaunchKernelGGL((k_nearT<T>), dim3(nleaf), dim3(256), 0, s, leaves, dcol, D, x, layer, y, y2);
-}
-
-void launch_zero(double* a, long long n, hipStream_t s) {
-   int blocks = (int)std::min<long long>((n + 255) / 256, 4096);
-   if (blocks < 1) blocks = 1;
-   hipLaunchKernelGGL(k_zero, dim3(blocks), dim3(256), 0, s, a, n);
-}
-
-#define FSVD_INST(T)                                                                                           \
-   template void launch_far_translate<T>(int, const TgtDesc*, const int*, const int*, const void*, const void*,      \
-                                         void*, int, hipStream_t);                                                   \
-   template void launch_apply_stage<T>(int, const ApplyArgs&, hipStream_t);                                          \
-   template void launch_transpose_batched<T>(int, const TransDesc*, hipStream_t);                                    \
-   template void launch_farT_source<T>(int, int, const TgtDesc*, const T*, const T*, const double*, void*, int,       \
-                                       hipStream_t);                                                                  \
-   template void launch_farT_target<T>(int, int, const SrcDesc*, const T*, const T*, const void*, int, double*,     \
-                                       double*, int,                                                              \
-                                       hipStream_t);                                                                  \
-   template void launch_nearT<T>(int, const LeafDesc*, const int*, const T*, const double*, int, double*, double*,   \
-                                 hipStream_t);
+#define FSVD_INST(T)                                                  \
+   template void launch_apply_stage<T>(int, const ApplyArgs&, hipStream_t); \
+   template void launch_transpose_batched<T>(int, const TransDesc*, hipStream_t);
 FSVD_INST(float)
 FSVD_INST(double)
 

@@ -195,6 +195,22 @@ struct LeafU {
    int ld, r, w_off, pad_;
 };
 
+// Transposed apply, one output leaf (np > 0 panels from p0): the near-field
+// blocks that hold its panels as columns, nbr[nb0 .. nb0 + nn) with `rows`
+// rows in all, and the row-basis blocks of its source cubes, ublk[u0 .. u0 +
+// nu) (LeafU with u_off into the panel-major bases, at the leaf's first panel).
+// A leaf of more than LT_SLAB panels (their sums in LDS) has several.
+constexpr int LT_SLAB = 1024;
+struct LeafT {
+   int p0, np, nb0, nn, rows, u0, nu, pad_;
+};
+// p points from q0; the leaf's first column at d_off of the near-field array,
+// the next one 2p further; row0: rows of the leaf's list before this block.
+struct NearT {
+   long long d_off;
+   int q0, p, row0, pad_;
+};
+
 // Element-wise transpose job: dst (cols x rows, row-major) = src^T.
 struct TransDesc {
    const void* src;
@@ -250,6 +266,14 @@ struct ApplyArgs {
    int ncol = 1;
    long long cs_x = 0, cs_y = 0, cs_tpart = 0, cs_spec = 0, cs_acc = 0, cs_w = 0;
    long long spec_delta = 0, acc_delta = 0;
+   // transposed apply: stages 0 to 3 with one input vector (layers = 1), stage
+   // 5 the output of its leaves into y (single layer) and y2 (double layer),
+   // either one null if not wanted
+   int layers = 2;
+   int nleafT = 0, maxnpT = 0;
+   const LeafT* leavesT = nullptr;   // in launch order (XCD map), np = 0: idle block
+   const NearT* nbrT = nullptr;
+   double* y2 = nullptr;
    // single column: the region split fused into the leaf stage (output
    // sp_y[sp_out[k]] = y_k + sp_corr[k] xd[k] instead of y)
    const int* sp_out = nullptr;

@@ -615,43 +615,20 @@ static std::vector<int4> assign_pipe_blocks(const std::vector<int4>& tasks, cons
    return out;
 }
 
-void make_pipe(PipeDev& d, const std::vector<const TreeOp*>& ops, hipStream_t s, int mode, bool pair) {
-   std::vector<TpTile> tiles;
-   std::vector<TpOct> octs;
-   std::vector<long long> oacc;
-   std::vector<int> gsrc, gint;
-   std::vector<int4> tasks;
-   std::vector<double> cost;
-   for (const TreeOp* op : ops) {
-      const ApplyPlan& P = op->plan;
-      const PipeHost& H = P.pipe_h;
-      if (!P.Tsp32.p) throw std::runtime_error("pipelined translation needs the FP32 operator");
-      const int tb = (int)tiles.size(), ob = (int)octs.size(), ab = (int)oacc.size(), sb = (int)gsrc.size();
-      const int gb = (int)gint.size();
-      for (size_t i = 0; i < H.tiles.size(); i++) {
-         TpTile t = H.tiles[i];
-         t.T = (const float2*)P.Tsp32.p + H.t_off[i];
-         t.spec = (const float2*)P.spec.p;
-         t.acc = (float2*)P.acc.p;
-         t.src_off += sb;
-         tiles.push_back(t);
-      }
-      for (TpOct o : H.octs) {
-         o.int_off += gb;
-         o.acc_idx += ab;
-         octs.push_back(o);
-      }
-      oacc.insert(oacc.end(), H.oacc.begin(), H.oacc.end());
-      gsrc.insert(gsrc.end(), H.gsrc.begin(), H.gsrc.end());
-      gint.insert(gint.end(), H.gint.begin(), H.gint.end());
-      for (size_t i = 0; i < H.tasks.size(); i++) {
-         int4 t = H.tasks[i];
-         t.x += tb;
-         t.z += ob;
-         tasks.push_back(t);
-         cost.push_back(H.cost[i]);
-      }
+void make_pipe(PipeDev& d, const ApplyPlan& P, const float* Tsp, hipStream_t s, int mode, bool pair) {
+   const PipeHost& H = P.pipe_h;
+   if (!Tsp) throw std::runtime_error("pipelined translation needs the FP32 operator");
+   std::vector<TpTile> tiles(H.tiles);
+   for (size_t i = 0; i < tiles.size(); i++) {
+      tiles[i].T = (const float2*)Tsp + H.t_off[i];
+      tiles[i].spec = (const float2*)P.spec.p;
+      tiles[i].acc = (float2*)P.acc.p;
    }
+   std::vector<TpOct> octs(H.octs);
+   std::vector<long long> oacc(H.oacc);
+   std::vector<int> gsrc(H.gsrc), gint(H.gint);
+   std::vector<int4> tasks(H.tasks);
+   std::vector<double> cost(H.cost);
    if (pair) {
       // each run of tasks of one level and 8-bin chunk (consecutive, over
       // the level's tiles) becomes the run of its first 4-bin halves, then
@@ -695,10 +672,10 @@ void make_pipe(PipeDev& d, const std::vector<const TreeOp*>& ops, hipStream_t s,
       for (long long a : oacc) targets += a >= 0;
       for (const TpTile& t : tiles) nsrc += t.nsrc;
       std::fprintf(stderr,
-                   "[fftsvd setup] pipelined translation (%d tree(s)): %d tiles (%.1f targets, %.1f sources each), "
+                   "[fftsvd setup] pipelined translation: %d tiles (%.1f targets, %.1f sources each), "
                    "%d tasks on %d blocks, block cost max/mean %.3f, %.1f steps per octet, %.3f of target slots "
                    "used\n",
-                   (int)ops.size(), (int)tiles.size(), (double)targets / std::max<size_t>(tiles.size(), 1),
+                   (int)tiles.size(), (double)targets / std::max<size_t>(tiles.size(), 1),
                    (double)nsrc / std::max<size_t>(tiles.size(), 1), (int)tasks.size(), nblk, imb,
                    (double)steps / std::max<size_t>(octs.size(), 1),
                    (double)targets / std::max<size_t>(8 * octs.size(), 1));
@@ -762,7 +739,7 @@ static PipeParams pipe_params(TreeOp& op, hipStream_t s) {
    for (const PipeParams& c : cand) {
       build_translate_pipe(P, P.tr_lv, P.tr_tgt, P.tr_isrc, P.tr_itoff, c);
       PipeDev d;
-      make_pipe(d, {&op}, s, c.mode);
+      make_pipe(d, P, P.Tsp32.p, s, c.mode);
       launch_pipe(d, s);
       FSVD_CHECK(hipEventRecord(e0, s));
       for (int r = 0; r < 3; r++) launch_pipe(d, s);
@@ -1012,7 +989,7 @@ static void build_apply_plan(TreeOp& op, bool want32, hipStream_t s) {
       timing_mark("plan: FP32 copies, tuning", tm);
       build_translate_pipe(P, P.tr_lv, P.tr_tgt, P.tr_isrc, P.tr_itoff, pp);
       timing_mark("plan: pipe tiles", tm);
-      make_pipe(P.pipe, {&op}, s, pp.mode);
+      make_pipe(P.pipe, P, P.Tsp32.p, s, pp.mode);
       op.stats.pipe = pp;
       timing_mark("plan: pipelined translation", tm);
    }
@@ -1207,7 +1184,6 @@ std::unique_ptr<TreeOp> build_tree_op(const double* pan_cent, int npan, const Pa
       for (int d = 0; d < 3; d++) ptsT[3 * (size_t)k + d] = pts[3 * (size_t)t.pt_perm[k] + d];
    op.pts_tree.upload(ptsT, s);
    op.pan_perm.upload(t.pan_perm, s);
-   op.yfar.alloc(std::max(npt, npan) + 1);
 
    // ---------------- near field (Cube_fill_D, Cube.c:715-793) ----------------
    // on a host thread and stream of its own, beside the far-field levels
@@ -1609,13 +1585,6 @@ std::unique_ptr<TreeOp> build_tree_op(const double* pan_cent, int npan, const Pa
    timing_mark("interaction lists", tm);
    if (want32) {
       to_f32(op.D64, op.D32, s);
-      for (FarLevel& lv : op.levels) {
-         to_f32(lv.T64, lv.T32, s);
-         to_f32(lv.VT64, lv.VT32, s);
-         to_f32(lv.PV64, lv.PV32, s);
-         to_f32(lv.UT64, lv.UT32, s);
-         to_f32(lv.UTI64, lv.UTI32, s);
-      }
       op.have32 = true;
    }
    FSVD_CHECK(hipStreamSynchronize(s));
@@ -1628,22 +1597,17 @@ std::unique_ptr<TreeOp> build_tree_op(const double* pan_cent, int npan, const Pa
    return opp;
 }
 
-template <typename T>
-static ApplyArgs make_args(TreeOp& op, const double* xs, const double* xd, double* y) {
-   const bool f32 = std::is_same<T, float>::value;
-   ApplyPlan& P = op.plan;
-   ApplyArgs a;
+// The launch arguments that a plan determines.
+static ApplyArgs plan_args(ApplyPlan& P) {
+   ApplyArgs a{};
    a.nchunk = P.nchunk;
    a.nsrc = P.nsrc;
    a.ntgt = P.ntgt;
    a.nsrc_big = P.nsrc_big;
    a.ntgt_big = P.ntgt_big;
-   a.nleaf = op.nleaf;
    a.proj_maxcols = P.proj_maxcols;
    a.maxr_src = P.maxr_src;
    a.max_n = P.max_n;
-   a.maxm = op.maxm;
-   a.maxp = op.maxp;
    a.chunks = P.chunks.p;
    a.src = P.src.p;
    a.tgt = P.tgt.p;
@@ -1663,6 +1627,21 @@ static ApplyArgs make_args(TreeOp& op, const double* xs, const double* xd, doubl
    a.gtgt = P.gtgt.p;
    a.gsrc = P.gsrc.p;
    a.gint = P.gint.p;
+   a.tpart = P.tpart.p;
+   a.spec = P.spec.p;
+   a.acc = P.acc.p;
+   a.w = P.w.p;
+   return a;
+}
+
+template <typename T>
+static ApplyArgs make_args(TreeOp& op, const double* xs, const double* xd, double* y) {
+   const bool f32 = std::is_same<T, float>::value;
+   ApplyPlan& P = op.plan;
+   ApplyArgs a = plan_args(P);
+   a.nleaf = op.nleaf;
+   a.maxm = op.maxm;
+   a.maxp = op.maxp;
    a.nmap_leaf = P.nmap_leaf;
    a.map_leaf = P.map_leaf.p;
    a.leaves = op.leaves.p;
@@ -1674,10 +1653,6 @@ static ApplyArgs make_args(TreeOp& op, const double* xs, const double* xd, doubl
    a.UTI = f32 ? (const void*)P.UTI32.p : (const void*)P.UTI64.p;
    a.UT = f32 ? (const void*)P.UT32.p : (const void*)P.UT64.p;
    a.D = f32 ? (const void*)op.D32.p : (const void*)op.D64.p;
-   a.tpart = P.tpart.p;
-   a.spec = P.spec.p;
-   a.acc = P.acc.p;
-   a.w = P.w.p;
    a.xs = xs;
    a.xd = xd;
    a.y = y;
@@ -1768,7 +1743,7 @@ static void apply_part_batch_impl(TreeOp& op, int part, int ncol, const double* 
    a.spec_delta = (long long)((const char*)P.specB.p - (const char*)P.spec.p);
    a.acc_delta = (long long)((const char*)P.accB.p - (const char*)P.acc.p);
    if (std::is_same<T, float>::value && ncol >= 2 && part == 2) {
-      if (!P.pipe2.nblk && P.pipe.nblk) make_pipe(P.pipe2, {&op}, s, 0, true);
+      if (!P.pipe2.nblk && P.pipe.nblk) make_pipe(P.pipe2, P, P.Tsp32.p, s, 0, true);
       a.nblk_p2 = P.pipe2.nblk;
       a.range_p2 = P.pipe2.range.p;
       a.task_p2 = P.pipe2.tasks.p;
@@ -1810,89 +1785,274 @@ void tree_apply(TreeOp& op, int prec, const double* xs, const double* xd, double
    }
 }
 
-// The transposed apply's per-level descriptors and interaction lists
-// (each source cube receives from the target cubes of its list), built and
-// uploaded on the transposed apply's first use.
-static void transpose_lists(TreeOp& op, hipStream_t s) {
-   if (op.haveT) return;
+// The transposed apply's plan (TransPlan), made on its first use.
+static void build_trans_plan(TreeOp& op, hipStream_t s) {
+   if (op.trans) return;
+   auto tp = std::make_unique<TransPlan>();
+   ApplyPlan& P = tp->P;
    const Tree& t = op.tree;
-   for (FarLevel& lv : op.levels) {
-      lv.h_tgtT.assign(lv.h_src.size(), TgtDesc{});
-      lv.h_isrcT.clear();
-      lv.h_itoffT.clear();
-      size_t si = 0;
-      for (size_t i = 0; i < t.cubes.size(); i++) {
-         const Cube& c = t.cubes[i];
-         if (c.level != lv.level || op.cube_src_slot[i] < 0) continue;
-         TgtDesc& td = lv.h_tgtT[si];
-         std::memset(&td, 0, sizeof(td));
-         td.spec_slot = op.cube_src_slot[i];
-         td.int_off = (int)lv.h_isrcT.size();
+   const size_t L = op.levels.size();
+   constexpr int CHUNK = 4096, PROJ_MAXCOLS = 512;   // as the forward plan's
+   // target cubes project their points, point-major U in the place of VT
+   std::vector<ProjChunk> chunks;
+   std::vector<SrcPlan> src;
+   std::vector<TransDesc> tr;
+   long long ut_n = 0;
+   for (const FarLevel& lv : op.levels) ut_n += (long long)lv.UT64.n;
+   P.VTc64.alloc(std::max<long long>(ut_n, 1));
+   // source cubes receive: both layers' rows of PV in the place of UTI
+   std::vector<TgtPlan> tgt;
+   std::vector<std::vector<int>> lv_w(L);
+   std::vector<long long> lv_vt(L);
+   long long ut_b = 0, uti_b = 0, pv_b = 0, vt_b = 0, t_b = 0, spec_b = 0, acc_b = 0;
+   int tpart_n = 0, w_n = 0;
+   std::vector<std::vector<int>> cubes_of(L);   // the level's cubes with a source slot, in slot order
+   for (size_t li = 0; li < L; li++) cubes_of[li].assign(op.levels[li].h_src.size(), -1);
+   for (size_t i = 0; i < t.cubes.size(); i++)
+      if (op.cube_src_slot[i] >= 0) cubes_of[t.cubes[i].level - 2][op.cube_src_slot[i]] = (int)i;
+   for (size_t li = 0; li < L; li++) {
+      const FarLevel& lv = op.levels[li];
+      const int pst = tr_pst(lv.pad);
+      P.max_n = std::max(P.max_n, lv.n);
+      for (const TgtDesc& td : lv.h_tgt) {
+         SrcPlan sp;
+         sp.n = lv.n;
+         sp.r = td.r;
+         sp.part_off = tpart_n;
+         sp.nchunk = 0;
+         const int cpc = std::max(1, std::min(PROJ_MAXCOLS, CHUNK / td.r));
+         for (int c0 = 0; c0 < td.nq; c0 += cpc) {
+            ProjChunk c;
+            c.vt_off = ut_b + td.u_off + (long long)c0 * td.r;
+            c.p0 = td.q0 + c0;
+            c.ncol = std::min(cpc, td.nq - c0);
+            c.r = td.r;
+            c.out_off = tpart_n;
+            tpart_n += td.r;
+            chunks.push_back(c);
+            sp.nchunk++;
+            P.proj_maxcols = std::max(P.proj_maxcols, c.ncol);
+         }
+         sp.pv_off = uti_b + td.uti_off;
+         sp.spec_off = spec_b + (long long)td.spec_slot * pst;
+         src.push_back(sp);
+         P.maxr_src = std::max(P.maxr_src, td.r);
+         tr.push_back({lv.UT64.p + td.u_off, P.VTc64.p + ut_b + td.u_off, td.r, td.nq});
+      }
+      tp->lv.push_back({(int)tgt.size(), (int)lv.h_src.size(), lv.pad, pst, lv.ntgt, t_b / 2, spec_b});
+      lv_vt[li] = vt_b;
+      for (size_t k = 0; k < lv.h_src.size(); k++) {
+         const SrcDesc& sd = lv.h_src[k];
+         const Cube& c = t.cubes[cubes_of[li][k]];
+         TgtPlan g;
+         g.n = lv.n;
+         g.r = 2 * sd.r;
+         g.pad = lv.pad;
+         g.int_off = (int)tp->isrc.size();
+         g.w_off = w_n;
+         g.t_off = t_b / 2;
+         g.acc_off = acc_b + (long long)sd.spec_slot * pst;
+         g.uti_off = pv_b + sd.pv_off;
          for (int o : c.itr)
             if (op.cube_tgt_slot[o] >= 0) {
-               lv.h_isrcT.push_back(op.cube_tgt_slot[o]);
-               lv.h_itoffT.push_back(offset_code(c.idx, t.cubes[o].idx));
+               const long long so = spec_b + (long long)op.cube_tgt_slot[o] * pst;
+               if (so > 0x7fffffffLL) throw std::runtime_error("spectrum offsets exceed 32 bits");
+               tp->isrc.push_back((int)so);
+               tp->itoff.push_back(offset_code(c.idx, t.cubes[o].idx));
             }
-         td.nint = (int)lv.h_isrcT.size() - td.int_off;
-         si++;
+         g.nint = (int)tp->isrc.size() - g.int_off;
+         lv_w[li].push_back(w_n);
+         w_n += 2 * sd.r;
+         tgt.push_back(g);
       }
-      lv.src.upload(lv.h_src, s);
-      lv.tgt.upload(lv.h_tgt, s);
-      lv.tgtT.upload(lv.h_tgtT, s);
-      lv.isrcT.upload(lv.h_isrcT, s);
-      lv.itoffT.upload(lv.h_itoffT, s);
+      ut_b += (long long)lv.UT64.n;
+      uti_b += (long long)lv.UTI64.n;
+      pv_b += (long long)lv.PV64.n;
+      vt_b += (long long)lv.VT64.n;
+      t_b += 2LL * 343 * pst;
+      spec_b += (long long)lv.ntgt * pst;
+      acc_b += (long long)lv.nsrc * pst;
    }
+   {
+      DBuf<TransDesc> dtr;
+      dtr.upload(tr, s);
+      launch_transpose_batched<double>((int)tr.size(), dtr.p, s);
+      if (op.have32) to_f32(P.VTc64, P.VTc32, s);
+      FSVD_CHECK(hipStreamSynchronize(s));
+   }
+   P.nchunk = (int)chunks.size();
+   P.nsrc = (int)src.size();
+   tp->ntgt = (int)tgt.size();
+   P.chunks.upload(chunks, s);
+   auto big_first = [](auto v) {
+      std::stable_partition(v.begin(), v.end(), [](const auto& e) { return e.n != 4; });
+      return v;
+   };
+   P.nsrc_big = (int)std::count_if(src.begin(), src.end(), [](const SrcPlan& e) { return e.n != 4; });
+   P.ntgt_big = (int)std::count_if(tgt.begin(), tgt.end(), [](const TgtPlan& e) { return e.n != 4; });
+   P.src.upload(big_first(src), s);
+   for (int v = 0; v < 3; v++) {
+      // the rows of one layer alone, its w where both layers' plan has it
+      std::vector<TgtPlan> g(tgt);
+      if (v < 2)
+         for (TgtPlan& e : g) {
+            e.r /= 2;
+            e.uti_off += (long long)v * e.r * e.n * e.n * e.n;
+            e.w_off += v * e.r;
+         }
+      tp->tgt[v].upload(big_first(g), s);
+   }
+   tp->h_tgt = std::move(tgt);
+   P.tpart.alloc(std::max(tpart_n, 1));
+   P.spec.alloc(2 * std::max<long long>(spec_b, 1));
+   P.acc.alloc(2 * std::max<long long>(acc_b, 1));
+   P.w.alloc(std::max(w_n, 1));
+   // the bins between a spectrum's pad and its stride stay zero
+   FSVD_CHECK(hipMemsetAsync(P.spec.p, 0, sizeof(double) * P.spec.n, s));
+   FSVD_CHECK(hipMemsetAsync(P.acc.p, 0, sizeof(double) * P.acc.n, s));
+   // output leaves (those with panels, in panel order): the near-field blocks
+   // that hold their panels as columns, in block order
+   std::vector<LeafT> leaves;
+   std::vector<int> leaf_cube, panel_leaf(std::max(t.npan, 1), -1);
+   for (size_t i = 0; i < t.cubes.size(); i++)
+      if (t.cubes[i].leaf && t.cubes[i].np > 0) leaf_cube.push_back((int)i);
+   std::stable_sort(leaf_cube.begin(), leaf_cube.end(),
+                    [&](int a, int b) { return t.cubes[a].p0 < t.cubes[b].p0; });
+   for (size_t k = 0; k < leaf_cube.size(); k++) {
+      const Cube& c = t.cubes[leaf_cube[k]];
+      for (int p = c.p0; p < c.p0 + c.np; p++) panel_leaf[p] = (int)k;
+   }
+   std::vector<std::vector<NearT>> near(leaf_cube.size());
+   for (size_t i = 0; i < t.cubes.size(); i++) {
+      const int lf = op.cube_leaf[i];
+      if (lf < 0) continue;
+      const LeafDesc& B = op.h_leaves[lf];
+      for (int c = 0; c < B.m;) {
+         // a run of columns that are one leaf's panels from its first on
+         const int pan = op.h_dcol[B.col_off + c], k = panel_leaf[pan];
+         const Cube& o = t.cubes[leaf_cube[k]];
+         if (o.p0 != pan || c + o.np > B.m) throw std::runtime_error("near-field columns are not whole leaves");
+         NearT e;
+         e.d_off = B.d_off + 2LL * B.p * c;
+         e.q0 = B.q0;
+         e.p = B.p;
+         e.row0 = 0;
+         e.pad_ = 0;
+         near[k].push_back(e);
+         c += o.np;
+      }
+   }
+   std::vector<NearT> nbr;
+   std::vector<LeafU> ublk;
+   std::vector<double> work;
+   for (size_t k = 0; k < leaf_cube.size(); k++) {
+      const Cube& c = t.cubes[leaf_cube[k]];
+      for (int j0 = 0; j0 < c.np; j0 += LT_SLAB) {
+         LeafT l;
+         l.p0 = c.p0 + j0;
+         l.np = std::min(LT_SLAB, c.np - j0);
+         l.nb0 = (int)nbr.size();
+         l.rows = 0;
+         l.pad_ = 0;
+         for (NearT e : near[k]) {
+            e.row0 = l.rows;
+            e.d_off += 2LL * e.p * j0;
+            l.rows += e.p;
+            nbr.push_back(e);
+         }
+         l.nn = (int)nbr.size() - l.nb0;
+         l.u0 = (int)ublk.size();
+         for (int a = leaf_cube[k]; a >= 0 && t.cubes[a].level >= 2; a = t.cubes[a].parent) {
+            const int li = t.cubes[a].level - 2, slot = op.cube_src_slot[a];
+            if (li >= (int)L || slot < 0) continue;
+            const SrcDesc& sd = op.levels[li].h_src[slot];
+            LeafU u;
+            u.u_off = lv_vt[li] + sd.vt_off + (long long)(l.p0 - sd.p0) * sd.r;
+            u.ld = sd.r;
+            u.r = sd.r;
+            u.w_off = lv_w[li][slot];
+            u.pad_ = 0;
+            ublk.push_back(u);
+         }
+         l.nu = (int)ublk.size() - l.u0;
+         leaves.push_back(l);
+         work.push_back(2.0 * l.np * l.rows + 64.0);
+         tp->maxnp = std::max(tp->maxnp, l.np);
+      }
+   }
+   std::vector<LeafT> ordered;
+   for (int k : xcd_block_map(work)) ordered.push_back(k >= 0 ? leaves[k] : LeafT{});
+   tp->nleaf = (int)ordered.size();
+   tp->leaves.upload(ordered, s);
+   tp->nbr.upload(nbr, s);
+   tp->ublk.upload(ublk, s);
    FSVD_CHECK(hipStreamSynchronize(s));
-   op.haveT = true;
+   op.trans = std::move(tp);
 }
 
-// y2 set: both layers from one pass (single layer into y, double into y2)
+bool tree_transpose_ready(const TreeOp& op, int prec) {
+   return op.trans && (prec == PREC_F32 ? op.trans->have32 : op.trans->have64);
+}
+
+void tree_prepare_transpose(TreeOp& op, int prec, hipStream_t s) {
+   if (tree_transpose_ready(op, prec)) return;
+   double tm = now_ms();
+   build_trans_plan(op, s);
+   timing_mark("transposed plan", tm);
+   TransPlan& tp = *op.trans;
+   if (prec == PREC_F32) {
+      if (!op.have32) throw std::runtime_error("operator has no FP32 copy");
+      build_translate_pipe(tp.P, tp.lv, tp.h_tgt, tp.isrc, tp.itoff, op.stats.pipe);
+      make_pipe(tp.P.pipe, tp.P, op.plan.Tsp32.p, s, op.stats.pipe.mode);
+      tp.have32 = true;
+   } else {
+      build_translate_f64(tp.P, tp.lv, tp.h_tgt, tp.isrc, tp.itoff, s);
+      tp.have64 = true;
+   }
+   timing_mark("transposed translation", tm);
+}
+
+// y = S^T x and y2 = D^T x, either one null if not wanted
 template <typename T>
-static void applyT_impl(TreeOp& op, int layer, const double* x, double* y, hipStream_t s, double* y2 = nullptr) {
+static void applyT_impl(TreeOp& op, const double* x, double* y, double* y2, hipStream_t s) {
    const bool f32 = std::is_same<T, float>::value;
-   transpose_lists(op, s);
-   for (FarLevel& lv : op.levels)
-      if (!lv.specT.p) {
-         lv.specT.alloc(2 * (size_t)std::max(1, lv.ntgt) * lv.pad);
-         lv.accT.alloc(2 * (size_t)std::max(1, lv.nsrc) * lv.pad);
-      }
-   launch_zero(y, op.tree.npan, s);
-   if (y2) launch_zero(y2, op.tree.npan, s);
-   for (FarLevel& lv : op.levels)
-      if (lv.ntgt)
-         launch_farT_source<T>(lv.n, lv.ntgt, lv.tgt.p, f32 ? (const T*)lv.UT32.p : (const T*)lv.UT64.p,
-                               f32 ? (const T*)lv.UTI32.p : (const T*)lv.UTI64.p, x, lv.specT.p, lv.maxr_tgt, s);
-   for (FarLevel& lv : op.levels)
-      if (lv.nsrc)
-         launch_far_translate<T>(lv.nsrc, lv.tgtT.p, lv.isrcT.p, lv.itoffT.p,
-                                 f32 ? (const void*)lv.T32.p : (const void*)lv.T64.p, lv.specT.p, lv.accT.p, lv.pad,
-                                 s);
-   for (FarLevel& lv : op.levels)
-      if (lv.nsrc)
-         launch_farT_target<T>(lv.n, lv.nsrc, lv.src.p, f32 ? (const T*)lv.VT32.p : (const T*)lv.VT64.p,
-                               f32 ? (const T*)lv.PV32.p : (const T*)lv.PV64.p, lv.accT.p, layer, y, y2, lv.maxr_src,
-                               s);
-   if (op.nleaf)
-      launch_nearT<T>(op.nleaf, op.leaves.p, op.dcol.p, f32 ? (const T*)op.D32.p : (const T*)op.D64.p, x, layer, y, y2,
-                      s);
+   tree_prepare_transpose(op, f32 ? PREC_F32 : PREC_F64, s);
+   TransPlan& tp = *op.trans;
+   ApplyPlan& P = tp.P;
+   const ApplyPlan& F = op.plan;
+   ApplyArgs a = plan_args(P);
+   a.layers = 1;
+   a.ntgt = tp.ntgt;
+   a.tgt = tp.tgt[y && y2 ? 2 : (y2 ? 1 : 0)].p;
+   a.VTc = f32 ? (const void*)P.VTc32.p : (const void*)P.VTc64.p;
+   a.PV = f32 ? (const void*)F.UTI32.p : (const void*)F.UTI64.p;
+   a.Tsp = f32 ? (const void*)F.Tsp32.p : (const void*)F.Tsp64.p;
+   a.UTI = f32 ? (const void*)F.PV32.p : (const void*)F.PV64.p;
+   a.xs = x;
+   for (int stage = 0; stage < 4; stage++) launch_apply_stage<T>(stage, a, s);
+   a.VTc = f32 ? (const void*)F.VTc32.p : (const void*)F.VTc64.p;
+   a.D = f32 ? (const void*)op.D32.p : (const void*)op.D64.p;
+   a.ublk = tp.ublk.p;
+   a.nleafT = tp.nleaf;
+   a.maxnpT = tp.maxnp;
+   a.leavesT = tp.leaves.p;
+   a.nbrT = tp.nbr.p;
+   a.y = y;
+   a.y2 = y2;
+   launch_apply_stage<T>(5, a, s);
 }
 
 void tree_apply_transpose_both(TreeOp& op, int prec, const double* x, double* ys, double* yd, hipStream_t s) {
    if (prec == PREC_F32) {
       if (!op.have32) throw std::runtime_error("operator has no FP32 copy");
-      applyT_impl<float>(op, 0, x, ys, s, yd);
+      applyT_impl<float>(op, x, ys, yd, s);
    } else {
-      applyT_impl<double>(op, 0, x, ys, s, yd);
+      applyT_impl<double>(op, x, ys, yd, s);
    }
 }
 
 void tree_apply_transpose(TreeOp& op, int prec, int layer, const double* x, double* y, hipStream_t s) {
-   if (prec == PREC_F32) {
-      if (!op.have32) throw std::runtime_error("operator has no FP32 copy");
-      applyT_impl<float>(op, layer, x, y, s);
-   } else {
-      applyT_impl<double>(op, layer, x, y, s);
-   }
+   tree_apply_transpose_both(op, prec, x, layer ? nullptr : y, layer ? y : nullptr, s);
 }
 
 }  // namespace fsvd

@@ -66,19 +66,10 @@ struct FarLevel {
    std::vector<SrcDesc> h_src;
    std::vector<TgtDesc> h_tgt;
    std::vector<int> h_isrc, h_itoff;     // target-side interaction lists
-   // the transposed apply's descriptors and lists (transposed: panel-side
-   // receivers, one per source cube), made on its first use
-   std::vector<TgtDesc> h_tgtT;
-   std::vector<int> h_isrcT, h_itoffT;
-   DBuf<SrcDesc> src;
-   DBuf<TgtDesc> tgt, tgtT;
-   DBuf<int> isrcT, itoffT;
    DBuf<double> T64;     // 343 * pad complex
-   DBuf<float> T32;
-   DBuf<double> specT, accT;     // ntgt*pad, nsrc*pad complex: transposed apply only, allocated on first use
-   // compressed blocks of this level (offsets in SrcDesc / TgtDesc)
+   // compressed blocks of this level (offsets in SrcDesc / TgtDesc); the apply
+   // plan holds the copies that the applies read, in both precisions
    DBuf<double> VT64, PV64, UT64, UTI64;
-   DBuf<float> VT32, PV32, UT32, UTI32;
 };
 
 // Parameters of the pipelined FP32 translation (the autotuner's choices):
@@ -173,6 +164,25 @@ struct ApplyPlan {
    DBuf<float> VTc32, PV32, Tsp32, UTI32, UT32;
 };
 
+// Transposed-apply plan of a tree, made on its first use: the forward stages
+// with the two sides swapped (point-major U for the projection, UTI in the
+// place of PV and PV in that of UTI, the interaction lists reversed), and the
+// output leaves.  The matrices other than U are the forward plan's.
+struct TransPlan {
+   ApplyPlan P;   // chunks, src, translation, work vectors, VTc = point-major U
+   DBuf<TgtPlan> tgt[3];   // the source cubes with the rows of the single layer, the double layer, both
+   int ntgt = 0;
+   // the translation's lists, for the plans made at the first use of each precision
+   std::vector<TrLevel> lv;
+   std::vector<TgtPlan> h_tgt;
+   std::vector<int> isrc, itoff;
+   bool have64 = false, have32 = false;
+   int nleaf = 0, maxnp = 0;   // nleaf: blocks of the leaf launch
+   DBuf<LeafT> leaves;         // in launch order
+   DBuf<NearT> nbr;
+   DBuf<LeafU> ublk;
+};
+
 // d/dkappa of a Yukawa operator at fixed tree, ranks and bases, in the
 // layouts of the FP64 apply plan: near-field blocks of the kappa-derivative
 // integrals, the derivatives of PV, of the T spectra and of UTI (VT and U
@@ -187,7 +197,6 @@ struct TreeOp {
    int kernel = LAPLACE;
    double kappa = 0.0;
    bool have32 = false;
-   bool haveT = false;   // the transposed apply's lists are on the device
    // geometry
    DBuf<double> pts_tree;     // tree-order point coordinates
    DBuf<int> pan_perm;        // tree order -> caller panel index
@@ -202,19 +211,18 @@ struct TreeOp {
    // far field
    std::vector<FarLevel> levels;
    std::vector<std::vector<double>> h_pinv;   // per level gp3 x 49 (levels >= 2)
-   DBuf<double> yfar;
    TreeOpStats stats;
    std::vector<int> cube_src_slot, cube_tgt_slot, cube_leaf;   // per cube: slot in its level / leaf index, -1
    ApplyPlan plan;
    std::unique_ptr<DkData> dk;
+   std::unique_ptr<TransPlan> trans;
 };
 
-// The device plan of one launch covering the FP32 translations of the given
-// trees (each with its own spectra), tasks dealt to the persistent blocks.
+// The device plan of one launch of plan P's FP32 translation (T spectra Tsp),
+// tasks dealt to the persistent blocks.
 // pair: the tasks of the two-column kernel (each 8-bin task split into its
 // two 4-bin halves, every level's first halves before its second halves).
-void make_pipe(PipeDev& d, const std::vector<const struct TreeOp*>& ops, hipStream_t s, int mode = 1,
-               bool pair = false);
+void make_pipe(PipeDev& d, const ApplyPlan& P, const float* Tsp, hipStream_t s, int mode = 1, bool pair = false);
 void launch_translate_pipe2(int nblk, const int2* range, const int4* tasks, const TpTile* tiles, const TpOct* octs,
                             const long long* oacc, const int* gsrc, const int* gint, hipStream_t s, int ncol,
                             long long sdel, long long adel, long long scs, long long acs);
@@ -266,6 +274,10 @@ void tree_batch_reserve(TreeOp& op, int ncol, hipStream_t s);
 // (FP64), y_t = S' xs + D' xd in tree order.
 void build_dkappa(TreeOp& op, const PanelGeom* d_panels, hipStream_t s);
 void tree_apply_dkappa(TreeOp& op, const double* xs, const double* xd, double* y, hipStream_t s);
+// The transposed apply's plan in one precision (made on its first use):
+// whether it is there, and made now, on stream s.
+bool tree_transpose_ready(const TreeOp& op, int prec);
+void tree_prepare_transpose(TreeOp& op, int prec, hipStream_t s);
 // y_t = A_layer^T x_t (panels, tree order).
 void tree_apply_transpose(TreeOp& op, int prec, int layer, const double* x, double* y, hipStream_t s);
 // Both layers at once, ys = S^T x and yd = D^T x: the points-side
@@ -278,25 +290,13 @@ void tree_apply_transpose_both(TreeOp& op, int prec, const double* x, double* ys
 std::vector<int> xcd_block_map(const std::vector<double>& work);
 
 // launchers (apply.hip / fill.hip)
-template <typename T>
-void launch_far_translate(int nblk, const TgtDesc* tgt, const int* isrc, const int* itoff, const void* Tspec,
-                          const void* spec, void* acc, int pad, hipStream_t s);
 // One stage of the forward apply (0 project, 1 source, 2 translate,
-// 3 target, 4 leaf) over every level of a tree.
+// 3 target, 4 leaf; 5 the output leaves of the transposed apply) over every
+// level of a tree.
 template <typename T>
 void launch_apply_stage(int stage, const ApplyArgs& a, hipStream_t s);
 template <typename T>
 void launch_transpose_batched(int n, const TransDesc* d, hipStream_t s);
-template <typename T>
-void launch_farT_source(int n, int nblk, const TgtDesc* tgt, const T* UT, const T* UTI, const double* x, void* spec,
-                        int maxr, hipStream_t s);
-template <typename T>
-void launch_farT_target(int n, int nblk, const SrcDesc* src, const T* VT, const T* PV, const void* acc, int layer,
-                        double* yfar, double* yfar2, int maxr, hipStream_t s);
-template <typename T>
-void launch_nearT(int nleaf, const LeafDesc* leaves, const int* dcol, const T* D, const double* x, int layer,
-                  double* y, double* y2, hipStream_t s);
-void launch_zero(double* a, long long n, hipStream_t s);
 void launch_integral_blocks(int nblk, const IntBlock* blocks, const double* bpts, const int* bpan,
                             const PanelGeom* panels, int kernel, double kappa, double* out, hipStream_t s);
 // Device panel geometry records: out[k] = record of panel ids[k] (panel k if

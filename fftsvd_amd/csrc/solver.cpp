@@ -646,24 +646,65 @@ static void qual_matvec(Problem& pr, int prec, const XT* x, double* y) {
    launch_qual_finish(n, pr.qual_perm.p, pr.qual_diag_t.p, R.xs.p, R.yt.p, 1.0 / fourpe, fourpe, c0, y, s);
 }
 
-// x = A^T y: per region (in order, on the library stream) the transposes
-// of k_split, the tree apply (both layers) and k_join, scatter-added into x
+// The transposed plans of the problem's operators, one host thread each.
+static void prepare_adjoint(Problem& pr, int prec) {
+   std::vector<Region*> todo;
+   for (Region& R : pr.regions) {
+      if (!R.op) continue;
+      if (prec == PREC_F32 && !R.op->have32) throw std::runtime_error("operator has no FP32 copy");
+      if (!tree_transpose_ready(*R.op, prec)) todo.push_back(&R);
+   }
+   if (todo.empty()) return;
+   int dev = 0;
+   FSVD_CHECK(hipGetDevice(&dev));
+   std::vector<std::exception_ptr> err(todo.size());
+   std::vector<std::thread> th;
+   for (size_t k = 0; k < todo.size(); k++)
+      th.emplace_back([&, k] {
+         try {
+            FSVD_CHECK(hipSetDevice(dev));
+            Region& R = *todo[k];
+            tree_prepare_transpose(*R.op, prec, R.lane == 0 ? pr.stream : pr.aux[R.lane - 1]);
+         } catch (...) {
+            err[k] = std::current_exception();
+         }
+      });
+   for (auto& t : th) t.join();
+   for (auto& e : err)
+      if (e) std::rethrow_exception(e);
+}
+
+// x = A^T y: per region the transposes of k_split and the tree apply (both
+// layers), the distinct operators on their matvec streams, then of k_join,
+// scatter-added into x region after region on the library stream
 // (SurfaceOperator_topmultiply transposed; Tree_multiply_transpose,
 // Tree.c:769-832, per layer).
 template <typename XT>
 static void adjoint_matvec(Problem& pr, int prec, const XT* y, double* x) {
    if (pr.qual) throw std::runtime_error("the adjoint of the qualocation operator is not provided");
    hipStream_t s = pr.stream;
-   FSVD_CHECK(hipMemsetAsync(x, 0, sizeof(double) * pr.nvec, s));
+   prepare_adjoint(pr, prec);
+   if (pr.naux > 0) {
+      FSVD_CHECK(hipEventRecord(pr.ev_fork, s));
+      for (int k = 0; k < pr.naux; k++) FSVD_CHECK(hipStreamWaitEvent(pr.aux[k], pr.ev_fork, 0));
+   }
    for (Region& R : pr.regions) {
       if (R.panel_ids.empty()) continue;
-      const int n = (int)R.panel_ids.size();
+      hipStream_t rs = R.lane == 0 ? s : pr.aux[R.lane - 1];
       TreeOp& op = R.shares_tree_with >= 0 ? *pr.regions[R.shares_tree_with].op : *R.op;
       if (prec == PREC_F32 && !op.have32) throw std::runtime_error("operator has no FP32 copy");
-      launch_gather_out<XT>(n, R.out_idx.p, y, R.yt.p, s);
-      tree_apply_transpose_both(op, prec, R.yt.p, R.xs.p, R.xd.p, s);
-      launch_scatter_adj(n, R.phi_idx.p, R.dphi_idx.p, R.s_phi.p, R.s_dphi.p, R.corr.p, R.yt.p, R.xs.p, R.xd.p, x, s);
+      launch_gather_out<XT>((int)R.panel_ids.size(), R.out_idx.p, y, R.yt.p, rs);
+      tree_apply_transpose_both(op, prec, R.yt.p, R.xs.p, R.xd.p, rs);
    }
+   FSVD_CHECK(hipMemsetAsync(x, 0, sizeof(double) * pr.nvec, s));
+   for (int k = 0; k < pr.naux; k++) {
+      FSVD_CHECK(hipEventRecord(pr.ev_join[k], pr.aux[k]));
+      FSVD_CHECK(hipStreamWaitEvent(s, pr.ev_join[k], 0));
+   }
+   for (Region& R : pr.regions)
+      if (!R.panel_ids.empty())
+         launch_scatter_adj((int)R.panel_ids.size(), R.phi_idx.p, R.dphi_idx.p, R.s_phi.p, R.s_dphi.p, R.corr.p,
+                            R.yt.p, R.xs.p, R.xd.p, x, s);
 }
 
 // Every region writes a disjoint set of rows of y (the phi rows of its own
