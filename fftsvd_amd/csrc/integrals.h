@@ -21,13 +21,15 @@
 
 namespace fsvd {
 
-__device__ __forceinline__ void laplace_integrals(const double* __restrict__ x, const PanelGeom& p, double& slp,
-                                                  double& dlp) {
+// The moment expansion: false if x is too close for it; xn, yn, zn: x in the
+// panel's frame.  Reads c, ax, mom and maxd of the panel only.
+__device__ __forceinline__ bool laplace_far(const double* __restrict__ x, const PanelGeom& p, double& xn, double& yn,
+                                            double& zn, double& slp, double& dlp) {
 #pragma clang fp contract(off)
    double r0 = x[0] - p.c[0], r1 = x[1] - p.c[1], r2 = x[2] - p.c[2];
-   double xn = p.ax[0] * r0 + p.ax[1] * r1 + p.ax[2] * r2;
-   double yn = p.ax[3] * r0 + p.ax[4] * r1 + p.ax[5] * r2;
-   double zn = p.ax[6] * r0 + p.ax[7] * r1 + p.ax[8] * r2;
+   xn = p.ax[0] * r0 + p.ax[1] * r1 + p.ax[2] * r2;
+   yn = p.ax[3] * r0 + p.ax[4] * r1 + p.ax[5] * r2;
+   zn = p.ax[6] * r0 + p.ax[7] * r1 + p.ax[8] * r2;
    double xsq = xn * xn, ysq = yn * yn, zsq = zn * zn;
    double rsq = xsq + ysq + zsq;
    double diagsq = p.maxd * p.maxd;
@@ -56,8 +58,15 @@ __device__ __forceinline__ void laplace_integrals(const double* __restrict__ x, 
       }
       slp = fs;
       dlp = fd;
-      return;
+      return true;
    }
+   return false;
+}
+
+// The closed form, x near the panel.
+__device__ __forceinline__ void laplace_near(const double* __restrict__ x, const PanelGeom& p, double xn, double yn,
+                                             double zn, double& slp, double& dlp) {
+#pragma clang fp contract(off)
    double za = fabs(zn);
    double xm[3], ym[3], fe[3], r[3];
    bool ok = true;
@@ -100,6 +109,12 @@ __device__ __forceinline__ void laplace_integrals(const double* __restrict__ x, 
    if (x[0] == p.c[0] && x[1] == p.c[1] && x[2] == p.c[2]) fd = 2.0 * M_PI;
    slp = fs;
    dlp = fd;
+}
+
+__device__ __forceinline__ void laplace_integrals(const double* __restrict__ x, const PanelGeom& p, double& slp,
+                                                  double& dlp) {
+   double xn, yn, zn;
+   if (!laplace_far(x, p, xn, yn, zn, slp, dlp)) laplace_near(x, p, xn, yn, zn, slp, dlp);
 }
 
 // Gauss-Legendre 4-point rule on [0,1] (closed form of the Golub-Welsch

@@ -426,80 +426,6 @@ __global__ void k_axpby(long long n, double a, const double* __restrict__ x, dou
       z[i] = a * x[i] + b * y[i];
 }
 
-// rhs[out[e]] = sum_i q_i / |x_i - c_e| over charges in order
-// (SurfaceOperator_makeRHS, SurfaceOperator.c:291-321).
-__global__ void k_rhs(int ne, const double* __restrict__ cent, const int* __restrict__ out, int nq,
-                      const double* __restrict__ qpos, const double* __restrict__ q, double* __restrict__ rhs) {
-   int e = blockIdx.x * blockDim.x + threadIdx.x;
-   if (e >= ne) return;
-   const double c0 = cent[3 * e], c1 = cent[3 * e + 1], c2 = cent[3 * e + 2];
-   double s = 0.0;
-   for (int i = 0; i < nq; i++) {
-      double qi = q[i];
-      if (qi == 0.0) continue;
-      double d0 = qpos[3 * i] - c0, d1 = qpos[3 * i + 1] - c1, d2 = qpos[3 * i + 2] - c2;
-      s += qi / sqrt(d0 * d0 + d1 * d1 + d2 * d2);
-   }
-   rhs[out[e]] += s;
-}
-
-// Many charge vectors (columns of q, nq x ncol) at once: the distances are
-// formed once per (element, charge); each column sums in charge order with
-// zero charges skipped, exactly as k_rhs, so column c equals k_rhs on q_c.
-constexpr int RHS_NB = 8;
-__global__ void k_rhs_batch(int ne, const double* __restrict__ cent, const int* __restrict__ out, int nq, int ncol,
-                            const double* __restrict__ qpos, const double* __restrict__ q, long long ldr,
-                            double* __restrict__ rhs) {
-   for (int e = blockIdx.x * blockDim.x + threadIdx.x; e < ne; e += gridDim.x * blockDim.x) {
-      const double c0 = cent[3 * e], c1 = cent[3 * e + 1], c2 = cent[3 * e + 2];
-      for (int col0 = 0; col0 < ncol; col0 += RHS_NB) {
-         double s[RHS_NB];
-#pragma unroll
-         for (int c = 0; c < RHS_NB; c++) s[c] = 0.0;
-         for (int i = 0; i < nq; i++) {
-            const double d0 = qpos[3 * i] - c0, d1 = qpos[3 * i + 1] - c1, d2 = qpos[3 * i + 2] - c2;
-            const double r = sqrt(d0 * d0 + d1 * d1 + d2 * d2);
-#pragma unroll
-            for (int c = 0; c < RHS_NB; c++) {
-               if (col0 + c < ncol) {
-                  const double qi = q[(long long)(col0 + c) * nq + i];
-                  if (qi != 0.0) s[c] += qi / r;
-               }
-            }
-         }
-#pragma unroll
-         for (int c = 0; c < RHS_NB; c++)
-            if (col0 + c < ncol) rhs[(long long)(col0 + c) * ldr + out[e]] += s[c];
-      }
-   }
-}
-
-// phi[j] += sum over panels of (a_e * slp - b_e * dlp) - (self ? 4 pi b_e : 0)
-// with Laplace integrals at the charge (direct branch of
-// SurfaceOperator_calculateReactionPotentials, SurfaceOperator.c:364-396).
-// For own panels a = sol[dphi], b = sol[phi], self check on; for child
-// panels a = -(eps_c/eps) sol[dphi_c], b = -sol[phi_c], self check off.
-__global__ void __launch_bounds__(256) k_potentials(int ne, const PanelGeom* __restrict__ panels,
-                                                    const int* __restrict__ pidx, const double* __restrict__ coef,
-                                                    const int* __restrict__ self_ok,
-                                                    const double* __restrict__ qpos, double* __restrict__ phi) {
-   __shared__ double red[8];
-   const int j = blockIdx.x;
-   const double x[3] = {qpos[3 * j], qpos[3 * j + 1], qpos[3 * j + 2]};
-   double s = 0.0;
-   for (int e = threadIdx.x; e < ne; e += blockDim.x) {
-      const PanelGeom& P = panels[pidx[e]];
-      double sl, dl;
-      laplace_integrals(x, P, sl, dl);
-      double a = coef[2 * e], b = coef[2 * e + 1];
-      double v = a * sl - b * dl;
-      if (self_ok[e] && x[0] == P.c[0] && x[1] == P.c[1] && x[2] == P.c[2]) v -= 4.0 * M_PI * b;
-      s += v;
-   }
-   s = block_sum(s, red);
-   if (threadIdx.x == 0) phi[j] += s;
-}
-
 // Qualocation operator (Solv_ecf_multiply_qual, GMRES.c:159-181), around
 // the transposed double-layer tree apply in tree order:
 //   gather: xa[k] = area_t[k] * x[perm[k]]
@@ -529,132 +455,6 @@ __global__ void k_qual_finish(int n, const int* __restrict__ perm, const double*
 // Diagonal preconditioner solve, x = b / p (x may alias b).
 __global__ void k_diag_div(int n, const double* __restrict__ p, const double* b, double* x) {
    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) x[i] = b[i] / p[i];
-}
-
-// Qualocation right-hand side (Charge_makerhs_ecf_qual, Charge.c:129-142):
-// rhs[i] = sum_j -dlp(charge j, panel i) q_j / (4 pi eps_in), in charge order.
-__global__ void __launch_bounds__(256) k_qual_rhs(int n, const PanelGeom* __restrict__ panels, int nq,
-                                                  const double* __restrict__ qpos, const double* __restrict__ q,
-                                                  double fourpe, double* __restrict__ rhs) {
-   for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
-      const PanelGeom& P = panels[i];
-      double r = 0.0;
-      for (int j = 0; j < nq; j++) {
-         const double x[3] = {qpos[3 * j], qpos[3 * j + 1], qpos[3 * j + 2]};
-         double sl, dl;
-         laplace_integrals(x, P, sl, dl);
-         r += -dl * q[j] / fourpe;
-      }
-      rhs[i] = r;
-   }
-}
-
-// k_potentials for ncol solution columns: coef holds (a, b) per element and
-// column (column-major, 2*ne per column); the integrals are formed once per
-// (charge, panel) and each column is summed and reduced as k_potentials.
-constexpr int POT_NB = 8;
-__global__ void __launch_bounds__(256) k_potentials_batch(int ne, int ncol, const PanelGeom* __restrict__ panels,
-                                                          const int* __restrict__ pidx,
-                                                          const double* __restrict__ coef,
-                                                          const int* __restrict__ self_ok,
-                                                          const double* __restrict__ qpos, int nq,
-                                                          double* __restrict__ phi) {
-   __shared__ double red[8];
-   const int j = blockIdx.x;
-   const double x[3] = {qpos[3 * j], qpos[3 * j + 1], qpos[3 * j + 2]};
-   for (int col0 = 0; col0 < ncol; col0 += POT_NB) {
-      double s[POT_NB];
-#pragma unroll
-      for (int c = 0; c < POT_NB; c++) s[c] = 0.0;
-      for (int e = threadIdx.x; e < ne; e += blockDim.x) {
-         const PanelGeom& P = panels[pidx[e]];
-         double sl, dl;
-         laplace_integrals(x, P, sl, dl);
-         const bool self = self_ok[e] && x[0] == P.c[0] && x[1] == P.c[1] && x[2] == P.c[2];
-#pragma unroll
-         for (int c = 0; c < POT_NB; c++) {
-            if (col0 + c < ncol) {
-               const double* cf = coef + (long long)(col0 + c) * 2 * ne;
-               const double a = cf[2 * e], b = cf[2 * e + 1];
-               double v = a * sl - b * dl;
-               if (self) v -= 4.0 * M_PI * b;
-               s[c] += v;
-            }
-         }
-      }
-#pragma unroll
-      for (int c = 0; c < POT_NB; c++) {
-         if (col0 + c < ncol) {   // uniform over the block
-            const double t = block_sum(s[c], red);
-            if (threadIdx.x == 0) phi[(long long)(col0 + c) * nq + j] += t;
-         }
-      }
-   }
-}
-
-// k_qual_rhs for ncol charge columns (q nq x ncol), columns of rhs ldr apart
-__global__ void __launch_bounds__(256) k_qual_rhs_batch(int n, const PanelGeom* __restrict__ panels, int nq, int ncol,
-                                                        const double* __restrict__ qpos, const double* __restrict__ q,
-                                                        double fourpe, long long ldr, double* __restrict__ rhs) {
-   for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
-      const PanelGeom& P = panels[i];
-      for (int col0 = 0; col0 < ncol; col0 += RHS_NB) {
-         double r[RHS_NB];
-#pragma unroll
-         for (int c = 0; c < RHS_NB; c++) r[c] = 0.0;
-         for (int j = 0; j < nq; j++) {
-            const double x[3] = {qpos[3 * j], qpos[3 * j + 1], qpos[3 * j + 2]};
-            double sl, dl;
-            laplace_integrals(x, P, sl, dl);
-#pragma unroll
-            for (int c = 0; c < RHS_NB; c++)
-               if (col0 + c < ncol) r[c] += -dl * q[(long long)(col0 + c) * nq + j] / fourpe;
-         }
-#pragma unroll
-         for (int c = 0; c < RHS_NB; c++)
-            if (col0 + c < ncol) rhs[(long long)(col0 + c) * ldr + i] = r[c];
-      }
-   }
-}
-
-// Transposed collection: per element e (a panel of a charged region) the
-// sums over charges of q_j slp(j, e) and q_j dlp(j, e), with the 4 pi
-// self term of k_potentials counted when the charge sits at the centroid.
-__global__ void __launch_bounds__(256) k_collect_t(int ne, const PanelGeom* __restrict__ panels,
-                                                   const int* __restrict__ pidx, const int* __restrict__ self_ok,
-                                                   int nq, const double* __restrict__ qpos,
-                                                   const double* __restrict__ q, double* __restrict__ ssl,
-                                                   double* __restrict__ sdl) {
-   for (int e = blockIdx.x * blockDim.x + threadIdx.x; e < ne; e += gridDim.x * blockDim.x) {
-      const PanelGeom& P = panels[pidx[e]];
-      double a = 0.0, b = 0.0;
-      for (int j = 0; j < nq; j++) {
-         const double x[3] = {qpos[3 * j], qpos[3 * j + 1], qpos[3 * j + 2]};
-         double sl, dl;
-         laplace_integrals(x, P, sl, dl);
-         a += q[j] * sl;
-         b += q[j] * dl;
-         if (self_ok[e] && x[0] == P.c[0] && x[1] == P.c[1] && x[2] == P.c[2]) b += 4.0 * M_PI * q[j];
-      }
-      ssl[e] = a;
-      sdl[e] = b;
-   }
-}
-
-// Transposed right-hand side: g[j] += sum_e lam[out[e]] / |c_e - x_j|.
-__global__ void __launch_bounds__(256) k_rhs_t(int ne, const double* __restrict__ cent, const int* __restrict__ out,
-                                               const double* __restrict__ lam, const double* __restrict__ qpos,
-                                               double* __restrict__ g) {
-   __shared__ double red[8];
-   const int j = blockIdx.x;
-   const double x0 = qpos[3 * j], x1 = qpos[3 * j + 1], x2 = qpos[3 * j + 2];
-   double s = 0.0;
-   for (int e = threadIdx.x; e < ne; e += blockDim.x) {
-      const double d0 = x0 - cent[3 * e], d1 = x1 - cent[3 * e + 1], d2 = x2 - cent[3 * e + 2];
-      s += lam[out[e]] / sqrt(d0 * d0 + d1 * d1 + d2 * d2);
-   }
-   s = block_sum(s, red);
-   if (threadIdx.x == 0) g[j] += s;
 }
 
 // diagonal of the near-field blocks: diag[p0 + i] from leaf rows i < p
@@ -855,29 +655,6 @@ void launch_qual_finish(int n, const int* perm, const double* diag_t, const doub
 void launch_diag_div(int n, const double* p, const double* b, double* x, hipStream_t s) {
    if (n > 0) hipLaunchKernelGGL(k_diag_div, dim3(nblocks(n)), dim3(256), 0, s, n, p, b, x);
 }
-void launch_qual_rhs(int n, const PanelGeom* panels, int nq, const double* qpos, const double* q, double fourpe,
-                     double* rhs, hipStream_t s) {
-   if (n > 0) hipLaunchKernelGGL(k_qual_rhs, dim3(nblocks(n)), dim3(256), 0, s, n, panels, nq, qpos, q, fourpe, rhs);
-}
-
-void launch_rhs_batch(int ne, const double* cent, const int* out, int nq, int ncol, const double* qpos,
-                      const double* q, long long ldr, double* rhs, hipStream_t s) {
-   if (ne > 0 && ncol > 0)
-      hipLaunchKernelGGL(k_rhs_batch, dim3(nblocks(ne)), dim3(256), 0, s, ne, cent, out, nq, ncol, qpos, q, ldr, rhs);
-}
-void launch_potentials_batch(int nq, int ne, int ncol, const PanelGeom* panels, const int* pidx, const double* coef,
-                             const int* self_ok, const double* qpos, double* phi, hipStream_t s) {
-   if (nq > 0 && ne > 0 && ncol > 0)
-      hipLaunchKernelGGL(k_potentials_batch, dim3(nq), dim3(256), 0, s, ne, ncol, panels, pidx, coef, self_ok, qpos,
-                         nq, phi);
-}
-void launch_qual_rhs_batch(int n, const PanelGeom* panels, int nq, int ncol, const double* qpos, const double* q,
-                           double fourpe, long long ldr, double* rhs, hipStream_t s) {
-   if (n > 0 && ncol > 0)
-      hipLaunchKernelGGL(k_qual_rhs_batch, dim3(nblocks(n)), dim3(256), 0, s, n, panels, nq, ncol, qpos, q, fourpe,
-                         ldr, rhs);
-}
-
 template <typename XT>
 void launch_gather_out(int n, const int* out_idx, const XT* y, double* yh, hipStream_t s) {
    if (n > 0) hipLaunchKernelGGL((k_gather_out<XT>), dim3(nblocks(n)), dim3(256), 0, s, n, out_idx, y, yh);
@@ -893,17 +670,6 @@ void launch_precond_t(int nb, const int* ia, const int* ib, const double* M, con
                       hipStream_t s) {
    if (nb > 0) hipLaunchKernelGGL(k_precond_t, dim3(nblocks(nb)), dim3(256), 0, s, nb, ia, ib, M, b, x);
 }
-void launch_collect_t(int ne, const PanelGeom* panels, const int* pidx, const int* self_ok, int nq, const double* qpos,
-                      const double* q, double* ssl, double* sdl, hipStream_t s) {
-   if (ne > 0)
-      hipLaunchKernelGGL(k_collect_t, dim3(nblocks(ne)), dim3(256), 0, s, ne, panels, pidx, self_ok, nq, qpos, q, ssl,
-                         sdl);
-}
-void launch_rhs_t(int nq, int ne, const double* cent, const int* out, const double* lam, const double* qpos, double* g,
-                  hipStream_t s) {
-   if (nq > 0 && ne > 0) hipLaunchKernelGGL(k_rhs_t, dim3(nq), dim3(256), 0, s, ne, cent, out, lam, qpos, g);
-}
-
 #define FSVD_KRYLOV_INST(VT)                                                                                        \
    template void launch_multidot<VT>(long long, int, int, const VT* const*, const double*, double*, hipStream_t); \
    template void launch_multiaxpy<VT>(long long, int, const double*, const VT* const*, double*, double*,          \
@@ -917,15 +683,6 @@ FSVD_KRYLOV_INST(double)
 FSVD_KRYLOV_INST(float)
 void launch_axpby(long long n, double a, const double* x, double b, const double* y, double* z, hipStream_t s) {
    hipLaunchKernelGGL(k_axpby, dim3(nblocks(n, 256, 4096)), dim3(256), 0, s, n, a, x, b, y, z);
-}
-void launch_rhs(int ne, const double* cent, const int* out, int nq, const double* qpos, const double* q, double* rhs,
-                hipStream_t s) {
-   if (ne > 0) hipLaunchKernelGGL(k_rhs, dim3(nblocks(ne)), dim3(256), 0, s, ne, cent, out, nq, qpos, q, rhs);
-}
-void launch_potentials(int nq, int ne, const PanelGeom* panels, const int* pidx, const double* coef,
-                       const int* self_ok, const double* qpos, double* phi, hipStream_t s) {
-   if (nq > 0 && ne > 0)
-      hipLaunchKernelGGL(k_potentials, dim3(nq), dim3(256), 0, s, ne, panels, pidx, coef, self_ok, qpos, phi);
 }
 void launch_leaf_diag(int nleaf, const LeafDesc* leaves, const double* D, double* ds, double* dd, hipStream_t s) {
    if (nleaf > 0) hipLaunchKernelGGL(k_leaf_diag, dim3(nleaf), dim3(64), 0, s, nleaf, leaves, D, ds, dd);

@@ -51,10 +51,6 @@ template <typename VT>
 void launch_cgs2_b(long long n, int m, int nch, int ncol, const GmDev* d, hipStream_t s);
 template <typename VT>
 void launch_normalize_givens_b(long long n, int np, int i, int W, int ncol, const GmDev* d, hipStream_t s);
-void launch_rhs(int ne, const double* cent, const int* out, int nq, const double* qpos, const double* q, double* rhs,
-                hipStream_t s);
-void launch_potentials(int nq, int ne, const PanelGeom* panels, const int* pidx, const double* coef,
-                       const int* self_ok, const double* qpos, double* phi, hipStream_t s);
 void launch_leaf_diag(int nleaf, const LeafDesc* leaves, const double* D, double* ds, double* dd, hipStream_t s);
 template <typename XT>
 void launch_qual_gather(int n, const int* perm, const double* area_t, const XT* x, double* xa, hipStream_t s);
@@ -67,18 +63,19 @@ void launch_scatter_adj(int n, const int* pi, const int* di, const double* sp, c
                         const double* yh, const double* vs, const double* vd, double* x, hipStream_t s);
 void launch_precond_t(int nb, const int* ia, const int* ib, const double* M, const double* b, double* x,
                       hipStream_t s);
+
+// sums over charges and panels, ncol columns at once; ws: room for partial
+// sums, which has to live until s has drained
+void launch_rhs(int ne, const double* cent, const int* out, int nq, int ncol, const double* qpos, const double* q,
+                long long ldr, double* rhs, DBuf<double>& ws, hipStream_t s);
+void launch_qual_rhs(int n, const PanelGeom* panels, int nq, int ncol, const double* qpos, const double* q,
+                     double fourpe, long long ldr, double* rhs, DBuf<double>& ws, hipStream_t s);
+void launch_potentials(int nq, int ne, int ncol, const PanelGeom* panels, const int* pidx, const double* coef,
+                       const int* self_ok, const double* qpos, double* phi, DBuf<double>& ws, hipStream_t s);
 void launch_collect_t(int ne, const PanelGeom* panels, const int* pidx, const int* self_ok, int nq, const double* qpos,
-                      const double* q, double* ssl, double* sdl, hipStream_t s);
+                      const double* q, double* ssl, double* sdl, DBuf<double>& ws, hipStream_t s);
 void launch_rhs_t(int nq, int ne, const double* cent, const int* out, const double* lam, const double* qpos, double* g,
-                  hipStream_t s);
-void launch_rhs_batch(int ne, const double* cent, const int* out, int nq, int ncol, const double* qpos,
-                      const double* q, long long ldr, double* rhs, hipStream_t s);
-void launch_potentials_batch(int nq, int ne, int ncol, const PanelGeom* panels, const int* pidx, const double* coef,
-                             const int* self_ok, const double* qpos, double* phi, hipStream_t s);
-void launch_qual_rhs_batch(int n, const PanelGeom* panels, int nq, int ncol, const double* qpos, const double* q,
-                           double fourpe, long long ldr, double* rhs, hipStream_t s);
-void launch_qual_rhs(int n, const PanelGeom* panels, int nq, const double* qpos, const double* q, double fourpe,
-                     double* rhs, hipStream_t s);
+                  DBuf<double>& ws, hipStream_t s);
 
 namespace {
 double now_ms() {
@@ -783,8 +780,9 @@ void problem_rhs(Problem& pr, double* rhs) {
       return;
    }
    if (pr.qual) {
-      launch_qual_rhs(pr.ntotal, pr.regions[0].d_panels.p, (int)pr.q.size(), pr.d_qpos.p, pr.d_q.p,
-                      4.0 * M_PI * pr.eps_in, rhs, s);
+      DBuf<double> ws;
+      launch_qual_rhs(pr.ntotal, pr.regions[0].d_panels.p, (int)pr.q.size(), 1, pr.d_qpos.p, pr.d_q.p,
+                      4.0 * M_PI * pr.eps_in, pr.nvec, rhs, ws, s);
       FSVD_CHECK(hipStreamSynchronize(s));
       return;
    }
@@ -805,11 +803,11 @@ void problem_rhs(Problem& pr, double* rhs) {
             out.push_back(C.startdphi + j);
          }
       }
-      DBuf<double> dc;
+      DBuf<double> dc, ws;
       DBuf<int> dout;
       dc.upload(cent, s);
       dout.upload(out, s);
-      launch_rhs((int)out.size(), dc.p, dout.p, (int)pr.q.size(), pr.d_qpos.p, pr.d_q.p, rhs, s);
+      launch_rhs((int)out.size(), dc.p, dout.p, (int)pr.q.size(), 1, pr.d_qpos.p, pr.d_q.p, pr.nvec, rhs, ws, s);
       FSVD_CHECK(hipStreamSynchronize(s));
    }
 }
@@ -821,8 +819,9 @@ void problem_rhs_batch(Problem& pr, int ncol, const double* q, double* rhs) {
    hipStream_t s = pr.stream;
    const int nq = (int)pr.q.size();
    if (pr.qual) {
-      launch_qual_rhs_batch(pr.ntotal, pr.regions[0].d_panels.p, nq, ncol, pr.d_qpos.p, q, 4.0 * M_PI * pr.eps_in,
-                            pr.nvec, rhs, s);
+      DBuf<double> ws;
+      launch_qual_rhs(pr.ntotal, pr.regions[0].d_panels.p, nq, ncol, pr.d_qpos.p, q, 4.0 * M_PI * pr.eps_in,
+                      pr.nvec, rhs, ws, s);
       FSVD_CHECK(hipStreamSynchronize(s));
       return;
    }
@@ -842,11 +841,11 @@ void problem_rhs_batch(Problem& pr, int ncol, const double* q, double* rhs) {
             out.push_back(C.startdphi + j);
          }
       }
-      DBuf<double> dc;
+      DBuf<double> dc, ws;
       DBuf<int> dout;
       dc.upload(cent, s);
       dout.upload(out, s);
-      launch_rhs_batch((int)out.size(), dc.p, dout.p, nq, ncol, pr.d_qpos.p, q, pr.nvec, rhs, s);
+      launch_rhs((int)out.size(), dc.p, dout.p, nq, ncol, pr.d_qpos.p, q, pr.nvec, rhs, ws, s);
       FSVD_CHECK(hipStreamSynchronize(s));
    }
 }
@@ -1539,11 +1538,11 @@ void problem_potentials(Problem& pr, const double* sol, double* phi_out, bool us
          coef[2 * (size_t)i] = sol[i];
       }
       DBuf<int> dp, dsf;
-      DBuf<double> dc;
+      DBuf<double> dc, ws;
       dp.upload(pidx, s);
       dsf.upload(self, s);
       dc.upload(coef, s);
-      launch_potentials(nq, pr.ntotal, pr.regions[0].d_panels.p, dp.p, dc.p, dsf.p, pr.d_qpos.p, dphi.p, s);
+      launch_potentials(nq, pr.ntotal, 1, pr.regions[0].d_panels.p, dp.p, dc.p, dsf.p, pr.d_qpos.p, dphi.p, ws, s);
       FSVD_CHECK(hipStreamSynchronize(s));
    }
    for (Region& R : pr.regions) {
@@ -1583,11 +1582,11 @@ void problem_potentials(Problem& pr, const double* sol, double* phi_out, bool us
          }
       }
       DBuf<int> dp, dsf;
-      DBuf<double> dc;
+      DBuf<double> dc, ws;
       dp.upload(pidx, s);
       dsf.upload(self, s);
       dc.upload(coef, s);
-      launch_potentials(nq, (int)pidx.size(), dall, dp.p, dc.p, dsf.p, pr.d_qpos.p, dphi.p, s);
+      launch_potentials(nq, (int)pidx.size(), 1, dall, dp.p, dc.p, dsf.p, pr.d_qpos.p, dphi.p, ws, s);
       FSVD_CHECK(hipStreamSynchronize(s));
    }
    if (nq) FSVD_CHECK(hipMemcpyAsync(phi_out, dphi.p, sizeof(double) * nq, hipMemcpyDeviceToHost, s));
@@ -1607,11 +1606,11 @@ void problem_potentials_batch(Problem& pr, int ncol, const double* sol, double* 
    auto run = [&](const std::vector<int>& pidx, const std::vector<int>& self, const std::vector<double>& coef,
                   const PanelGeom* panels) {
       DBuf<int> dp, dsf;
-      DBuf<double> dc;
+      DBuf<double> dc, ws;
       dp.upload(pidx, s);
       dsf.upload(self, s);
       dc.upload(coef, s);
-      launch_potentials_batch(nq, (int)pidx.size(), ncol, panels, dp.p, dc.p, dsf.p, pr.d_qpos.p, dphi.p, s);
+      launch_potentials(nq, (int)pidx.size(), ncol, panels, dp.p, dc.p, dsf.p, pr.d_qpos.p, dphi.p, ws, s);
       FSVD_CHECK(hipStreamSynchronize(s));
    };
    if (pr.qual) {
@@ -1698,12 +1697,12 @@ static SolveInfo energy_adjoint(Problem& pr, int mode, const double* sol_host, d
          }
       const int ne = (int)pidx.size();
       DBuf<int> dp, dsf;
-      DBuf<double> dsl, ddl;
+      DBuf<double> dsl, ddl, ws;
       dp.upload(pidx, s);
       dsf.upload(self, s);
       dsl.alloc(std::max(ne, 1));
       ddl.alloc(std::max(ne, 1));
-      launch_collect_t(ne, dall, dp.p, dsf.p, nq, pr.d_qpos.p, pr.d_q.p, dsl.p, ddl.p, s);
+      launch_collect_t(ne, dall, dp.p, dsf.p, nq, pr.d_qpos.p, pr.d_q.p, dsl.p, ddl.p, ws, s);
       std::vector<double> ssl(ne), sdl(ne);
       FSVD_CHECK(hipMemcpyAsync(ssl.data(), dsl.p, sizeof(double) * ne, hipMemcpyDeviceToHost, s));
       FSVD_CHECK(hipMemcpyAsync(sdl.data(), ddl.p, sizeof(double) * ne, hipMemcpyDeviceToHost, s));
@@ -1755,11 +1754,11 @@ SolveInfo problem_grad_charges(Problem& pr, int mode, const double* sol_host, do
             out.push_back(C.startdphi + j);
          }
       }
-      DBuf<double> dc;
+      DBuf<double> dc, ws;
       DBuf<int> dout;
       dc.upload(cent, s);
       dout.upload(out, s);
-      launch_rhs_t(nq, (int)out.size(), dc.p, dout.p, dlam.p, pr.d_qpos.p, dgq.p, s);
+      launch_rhs_t(nq, (int)out.size(), dc.p, dout.p, dlam.p, pr.d_qpos.p, dgq.p, ws, s);
       FSVD_CHECK(hipStreamSynchronize(s));
    }
    std::vector<double> bt(std::max(nq, 1));
