@@ -547,8 +547,364 @@ __device__ void source_body(const SrcPlan& d, const T* __restrict__ tpart, const
    grid_forward<n, T>(g, A, B, spec + d.spec_off, cs, sn, gr);
 }
 
-// LDS of one source cube's work (block groups of nt threads; a wave group
-// of 64 lanes uses no partial-sum rows when GP3 = 64)
+// ---------------------------------------------------------------------------
+// Cubes of four grid points per side (N = 7, H = 4, 64 grid values), one per
+// wavefront.  What bounds grid_forward and grid_backward here is the LDS: three
+// reads per complex multiply-add (the value, the table's cosine and sine) and an
+// integer remainder for the table's index.  In these forms a lane makes a whole
+// line of the seven-point transform from values read once, with literal
+// twiddles; the other two dimensions take their four twiddles per lane from a
+// 7-entry table, once.  About 45 LDS operations per target cube instead of 160.
+// P columns side by side where a line's 28 lanes leave room for two.
+// Kernel times before and after: k_target 6.6 to 4.9 us (FP64, 1280 panels), 17.7
+// to 15.2 us (FP32, 30 000 panels; the other cubes bound it now), 70 to 62 us
+// (100 000; UTI from memory bounds it); 64 FP32 columns of 30 000 panels: target
+// 917 to 465 us a tree, source 575 to 407, of which the other cubes take 208
+// and 225.
+
+// e^{-2 pi i m / 7} = C7[m] - i S7[m]
+constexpr double C7[7] = {1.0,
+                          0.62348980185873353053,
+                          -0.22252093395631440429,
+                          -0.90096886790241912624,
+                          -0.90096886790241912624,
+                          -0.22252093395631440429,
+                          0.62348980185873353053};
+constexpr double S7[7] = {0.0,
+                          0.78183148246802980871,
+                          0.97492791218182360702,
+                          0.43388373911755812048,
+                          -0.43388373911755812048,
+                          -0.97492791218182360702,
+                          -0.78183148246802980871};
+
+template <typename T>
+__device__ __forceinline__ void table7(typename Cplx<T>::type* tw, int lane) {
+   T c = 1, sn = 0;
+#pragma unroll
+   for (int m = 1; m < 7; m++) {
+      c = lane == m ? (T)C7[m] : c;
+      sn = lane == m ? (T)S7[m] : sn;
+   }
+   if (lane < 7) {
+      tw[lane].x = c;
+      tw[lane].y = sn;
+   }
+}
+
+// v from lane ^ X, X a power of two below 16
+template <int CTRL>
+__device__ __forceinline__ float dpp_move(float v) {
+   return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, false));
+}
+template <int CTRL>
+__device__ __forceinline__ double dpp_move(double v) {
+   const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, 0xf, 0xf, false);
+   const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, 0xf, 0xf, false);
+   return __hiloint2double(hi, lo);
+}
+template <int X, typename T>
+__device__ __forceinline__ T lane_xor(T v) {
+   if constexpr (X == 8) return dpp_move<0x128>(v);                       // row rotate by 8
+   if constexpr (X == 4) return dpp_move<0x1B>(dpp_move<0x141>(v));       // ^7, then ^3 within quads
+   if constexpr (X == 2) return dpp_move<0x4E>(v);
+   return dpp_move<0xB1>(v);
+}
+
+// Sums of NV values over the 16 lanes of a row, in the order of a butterfly
+// over 8, 4, 2, 1; each step hands half of the values on while there are two or
+// more, so v[0] ends as the sum of value `lane15 / (16 / NV)`.
+template <int NV, int X, typename T>
+__device__ __forceinline__ void row_sums(T* v, int lane15) {
+   if constexpr (NV > 1) {
+      const bool up = lane15 & X;
+#pragma unroll
+      for (int k = 0; k < NV / 2; k++) {
+         const T give = up ? v[k] : v[k + NV / 2], mine = up ? v[k + NV / 2] : v[k];
+         v[k] = mine + lane_xor<X>(give);
+      }
+   } else {
+      v[0] += lane_xor<X>(v[0]);
+   }
+   if constexpr (X > 1) row_sums<(NV > 1 ? NV / 2 : 1), X / 2>(v, lane15);
+}
+
+// A source cube's spectra, columns 0 .. nc - 1 of the group: as source_body.
+template <typename T, bool NT, int NL, int NC>
+__device__ void source4(const SrcPlan& d, const T* __restrict__ tpart, long long cs_tpart, const T* __restrict__ PV,
+                        typename Cplx<T>::type* __restrict__ spec, long long cs_spec, int nc, unsigned char* smem,
+                        int lane) {
+   using C2 = typename Cplx<T>::type;
+   constexpr int P = NC > 1 ? 2 : 1;
+   T* g = (T*)smem;              // 64
+   C2* A = (C2*)(g + 64);        // 16 lines x 4
+   C2* B = A + 64;               // P x 28 lines x 4
+   C2* tw = B + 112 * P;         // 7
+   T* t = (T*)(tw + 8);          // NC x NL r: ts then td
+   const WaveGroup gr{lane};
+   const int R2 = NL * d.r;
+   // the first rows of PV travel while the chunk partials are summed
+   const T* pv = PV + d.pv_off + lane;
+   T v[8];
+#pragma unroll
+   for (int u = 0; u < 8; u++) v[u] = R2 ? ld_op<NT>(pv + (u < R2 ? u : 0) * 64) : (T)0;
+   table7<T>(tw, lane);
+#pragma unroll
+   for (int j = 0; j < NC; j++) {
+      if (j >= nc) break;
+      for (int k = lane; k < R2; k += 64) {
+         // in chunk order, eight loads in flight
+         const T* pp = tpart + j * cs_tpart + d.part_off + k;
+         T a = 0;
+         int i = 0;
+         for (; i + 7 < d.nchunk; i += 8) {
+            T q[8];
+#pragma unroll
+            for (int u = 0; u < 8; u++) q[u] = pp[(long long)(i + u) * R2];
+#pragma unroll
+            for (int u = 0; u < 8; u++) a += q[u];
+         }
+         if (i < d.nchunk) {
+            T q[7];
+#pragma unroll
+            for (int u = 0; u < 7; u++) q[u] = i + u < d.nchunk ? pp[(long long)(i + u) * R2] : (T)0;
+#pragma unroll
+            for (int u = 0; u < 7; u++)
+               if (i + u < d.nchunk) a += q[u];
+         }
+         t[j * R2 + k] = a;
+      }
+   }
+   gr.sync();
+   T a[NC][4];
+#pragma unroll
+   for (int j = 0; j < NC; j++)
+#pragma unroll
+      for (int u = 0; u < 4; u++) a[j][u] = 0;
+   int k = 0;
+   for (; k + 8 <= R2; k += 8) {
+      T x[8];
+#pragma unroll
+      for (int u = 0; u < 8; u++) x[u] = v[u];
+      // the next rows (past the last: its row again, unused)
+      if (k + 8 < R2)
+#pragma unroll
+         for (int u = 0; u < 8; u++) v[u] = ld_op<NT>(pv + (long long)min(k + 8 + u, R2 - 1) * 64);
+#pragma unroll
+      for (int j = 0; j < NC; j++) {
+         const T* tj = t + (j < nc ? j : 0) * R2 + k;
+#pragma unroll
+         for (int u = 0; u < 8; u++) a[j][u & 3] = fma(x[u], tj[u], a[j][u & 3]);
+      }
+   }
+   if (k < R2) {
+#pragma unroll
+      for (int j = 0; j < NC; j++) {
+         const T* tj = t + (j < nc ? j : 0) * R2 + k;
+#pragma unroll
+         for (int u = 0; u < 7; u++)
+            if (k + u < R2) a[j][u & 3] = fma(v[u], tj[u], a[j][u & 3]);
+      }
+   }
+   // twiddles of the first dimension (lane & 3 = c) and, for b = lane & 3
+   // and b + 4, of the second; all for points 2 .. 5 of the box
+   const int c4 = lane & 3;
+   C2 w0[4], w1[4];
+#pragma unroll
+   for (int k = 0; k < 4; k++) {
+      w0[k] = tw[(c4 * (k + 2)) % 7];
+      w1[k] = tw[((c4 + 4) * (k + 2)) % 7];
+   }
+#pragma unroll
+   for (int j0 = 0; j0 < NC; j0 += P) {
+      if (j0 >= nc) break;
+#pragma unroll
+      for (int p = 0; p < P; p++) {
+         if (j0 + p >= nc) break;
+         const int j = j0 + p;
+         g[lane] = (a[j][0] + a[j][1]) + (a[j][2] + a[j][3]);
+         gr.sync();
+         {
+            const T* row = g + (lane & ~3);
+            T re = 0, im = 0;
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+               re = fma(row[k], w0[k].x, re);
+               im = fma(-row[k], w0[k].y, im);
+            }
+            A[lane].x = re;   // (i, j, c)
+            A[lane].y = im;
+         }
+         gr.sync();
+         {
+            const int c = (lane >> 2) & 3, i = lane >> 4;
+            T r0 = 0, m0 = 0, r1 = 0, m1 = 0;
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+               const C2 z = A[(4 * i + k) * 4 + c];
+               r0 = fma(z.y, w0[k].y, fma(z.x, w0[k].x, r0));
+               m0 = fma(-z.x, w0[k].y, fma(z.y, w0[k].x, m0));
+               r1 = fma(z.y, w1[k].y, fma(z.x, w1[k].x, r1));
+               m1 = fma(-z.x, w1[k].y, fma(z.y, w1[k].x, m1));
+            }
+            C2* Bp = B + 112 * p + 28 * i + c;   // (i, b, c)
+            Bp[4 * c4].x = r0;
+            Bp[4 * c4].y = m0;
+            if (c4 < 3) {
+               Bp[4 * (c4 + 4)].x = r1;
+               Bp[4 * (c4 + 4)].y = m1;
+            }
+         }
+         gr.sync();
+      }
+      const int p = P > 1 && lane >= 28 ? 1 : 0, bc = lane - 28 * p;
+      if (bc < 28 && j0 + p < nc) {
+         C2 z[4];
+#pragma unroll
+         for (int i = 0; i < 4; i++) z[i] = B[112 * p + 28 * i + bc];
+         C2* o = spec + (j0 + p) * cs_spec + d.spec_off + bc;
+#pragma unroll
+         for (int m = 0; m < 7; m++) {
+            T re = 0, im = 0;
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+               const T cs = (T)C7[(m * (i + 2)) % 7], sn = (T)S7[(m * (i + 2)) % 7];
+               re = fma(z[i].y, sn, fma(z[i].x, cs, re));
+               im = fma(-z[i].x, sn, fma(z[i].y, cs, im));
+            }
+            C2 y;
+            y.x = re;
+            y.y = im;
+            o[28 * m] = y;
+         }
+      }
+      gr.sync();
+   }
+}
+
+template <typename T>
+__host__ __device__ constexpr size_t source4_lds(int maxr, int NC) {
+   return (sizeof(T) * (64 + 2 * (64 + 112 * (NC > 1 ? 2 : 1) + 8) + 2 * (size_t)maxr * NC) + 15) / 16 * 16;
+}
+
+// A target cube's w = UTI h, columns 0 .. nc - 1 of the group: as target_body,
+// each spectrum transformed straight from memory, each UTI row read once.
+template <typename T, int NC>
+__device__ void target4(const TgtPlan& d, const T* __restrict__ UTI, const typename Cplx<T>::type* __restrict__ acc,
+                        long long cs_acc, T* __restrict__ w, long long cs_w, int nc, unsigned char* smem, int lane) {
+   using C2 = typename Cplx<T>::type;
+   constexpr int P = NC > 1 ? 2 : 1, RU = NC > 1 ? 2 : 4, RP = 4 * RU, NV = NC * RU;
+   T* h = (T*)smem;             // NC x 64
+   C2* C1 = (C2*)(h + 64 * NC); // P x 28 lines x 4
+   C2* Cc = C1 + 112 * P;       // 16 lines x 4
+   C2* tw = Cc + 64;            // 7
+   const WaveGroup gr{lane};
+   const int kr = lane >> 4, ql = lane & 15;
+   const T* uti = UTI + d.uti_off + ql;
+   // RU rows per lane; of a single column the first ones travel during the
+   // transform (of several they would cost registers that the sums need)
+   T x[RU][4];
+   auto load_rows = [&](int k) {
+#pragma unroll
+      for (int u = 0; u < RU; u++) {
+         const T* row = uti + (long long)(k + 4 * u < d.r ? k + 4 * u : 0) * 64;
+#pragma unroll
+         for (int q = 0; q < 4; q++) x[u][q] = row[16 * q];
+      }
+   };
+   const int p = P > 1 && lane >= 28 ? 1 : 0, bc = lane - 28 * p;
+   C2 z[7];
+   auto load_line = [&](int j0) {
+      const C2* in = acc + (j0 + p < nc ? j0 + p : j0) * cs_acc + d.acc_off + (bc < 28 ? bc : 0);
+#pragma unroll
+      for (int m = 0; m < 7; m++) z[m] = in[28 * m];
+   };
+   load_line(0);
+   if (NC == 1 && kr < d.r) load_rows(kr);
+   table7<T>(tw, lane);
+   gr.sync();
+   // twiddles of point (lane & 3) + 2, for the second and third dimension
+   C2 wl[7];
+#pragma unroll
+   for (int b = 1; b < 7; b++) wl[b] = tw[(b * ((lane & 3) + 2)) % 7];
+#pragma unroll 1
+   for (int j0 = 0; j0 < NC && j0 < nc; j0 += P) {
+      if (bc < 28) {
+         C2* o = C1 + 112 * p + bc;   // (i, b, c)
+#pragma unroll
+         for (int i = 0; i < 4; i++) {
+            T re = 0, im = 0;
+#pragma unroll
+            for (int m = 0; m < 7; m++) {
+               const T cs = (T)C7[(m * (i + 2)) % 7], sn = (T)S7[(m * (i + 2)) % 7];
+               re = fma(-z[m].y, sn, fma(z[m].x, cs, re));
+               im = fma(z[m].x, sn, fma(z[m].y, cs, im));
+            }
+            o[28 * i].x = re;
+            o[28 * i].y = im;
+         }
+      }
+      if (j0 + P < nc) load_line(j0 + P);
+      gr.sync();
+#pragma unroll
+      for (int pp = 0; pp < P; pp++) {
+         if (j0 + pp >= nc) break;
+         {
+            const int c = (lane >> 2) & 3, i = lane >> 4;
+            const C2* in = C1 + 112 * pp + 28 * i + c;
+            T re = in[0].x, im = in[0].y;
+#pragma unroll
+            for (int b = 1; b < 7; b++) {
+               const C2 y = in[4 * b];
+               re = fma(-y.y, wl[b].y, fma(y.x, wl[b].x, re));
+               im = fma(y.x, wl[b].y, fma(y.y, wl[b].x, im));
+            }
+            C2 y;
+            y.x = re;
+            y.y = im;
+            Cc[16 * i + 4 * (lane & 3) + c] = y;   // (i, j, c)
+         }
+         gr.sync();
+         {
+            const C2* row = Cc + (lane & ~3);
+            T v = row[0].x;
+#pragma unroll
+            for (int c = 1; c < 4; c++) v = fma((T)2, fma(-row[c].y, wl[c].y, row[c].x * wl[c].x), v);
+            h[64 * (j0 + pp) + lane] = v * (T)(1.0 / 343.0);
+         }
+         gr.sync();
+      }
+   }
+   T hq[NC][4];
+#pragma unroll
+   for (int j = 0; j < NC; j++)
+#pragma unroll
+      for (int q = 0; q < 4; q++) hq[j][q] = h[64 * (j < nc ? j : 0) + 16 * q + ql];
+   for (int k = kr; k < d.r; k += RP) {
+      if (NC > 1) load_rows(k);
+      T s[NV];
+#pragma unroll
+      for (int j = 0; j < NC; j++)
+#pragma unroll
+         for (int u = 0; u < RU; u++) {
+            T a = x[u][0] * hq[j][0];
+#pragma unroll
+            for (int q = 1; q < 4; q++) a = fma(x[u][q], hq[j][q], a);
+            s[RU * j + u] = a;
+         }
+      if (NC == 1 && k + RP < d.r) load_rows(k + RP);
+      row_sums<NV, 8>(s, ql);
+      const int idx = ql / (16 / NV), j = idx / RU, row = k + 4 * (idx % RU);
+      if (ql % (16 / NV) == 0 && j < nc && row < d.r) w[j * cs_w + d.w_off + row] = s[0];
+   }
+}
+
+template <typename T>
+__host__ __device__ constexpr size_t target4_lds(int NC) {
+   return (sizeof(T) * (64 * NC + 2 * (112 * (NC > 1 ? 2 : 1) + 64 + 8)) + 15) / 16 * 16;
+}
+
+// LDS of one source cube's work (block groups of nt threads)
 template <typename T>
 __host__ __device__ constexpr size_t source_cube_lds(int n, int maxr, int nt) {
    return sizeof(typename Cplx<T>::type) * (size_t)(n * n * ((2 * n - 1) / 2 + 1) + n * (2 * n - 1) * ((2 * n - 1) / 2 + 1)) +
@@ -589,7 +945,26 @@ __global__ void __launch_bounds__(CUBE_NT) k_source(const SrcPlan* __restrict__ 
    const int wave = threadIdx.x >> 6, i = nbig + (cb.b - nbig) * (CUBE_NT / 64) + wave;
    if (i >= nsrc) return;
    const SrcPlan d = src[i];
-   source_body<4, T, NT, NL>(d, tpart, PV, spec, smem + (size_t)wave * wave_lds, WaveGroup{(int)(threadIdx.x & 63)});
+   source4<T, NT, NL, 1>(d, tpart, 0, PV, spec, 0, 1, smem + (size_t)wave * wave_lds, threadIdx.x & 63);
+}
+
+// Source cubes of four grid points per side for SRC_NC columns per wavefront
+// (LDS for two in FP64), which share each read of PV: read once per column from
+// L2 it was the bound, 0.35 ms per tree for 64 columns of 30 000 panels, now 0.18.
+template <typename T>
+constexpr int SRC_NC = sizeof(T) == 4 ? 4 : 2;
+template <typename T>
+__global__ void __launch_bounds__(CUBE_NT) k_source_mc(const SrcPlan* __restrict__ src, int nsrc,
+                                                       const T* __restrict__ tpart, const T* __restrict__ PV,
+                                                       typename Cplx<T>::type* __restrict__ spec, int wave_lds, int nb,
+                                                       int ncol, long long cs_tpart, long long cs_spec) {
+   extern __shared__ __align__(16) unsigned char smem[];
+   const ColBlk cb = col_block((ncol + SRC_NC<T> - 1) / SRC_NC<T>);
+   const int wave = threadIdx.x >> 6, i = cb.b * (CUBE_NT / 64) + wave, c0 = cb.c * SRC_NC<T>;
+   if (cb.b >= nb || i >= nsrc) return;
+   const SrcPlan d = src[i];
+   source4<T, false, 2, SRC_NC<T>>(d, tpart + c0 * cs_tpart, cs_tpart, PV, spec + c0 * cs_spec, cs_spec,
+                                min(SRC_NC<T>, ncol - c0), smem + (size_t)wave * wave_lds, threadIdx.x & 63);
 }
 
 // FP64 translation by tiles: a block owns BC frequency bins (one TR_ROW-byte
@@ -1420,7 +1795,7 @@ __host__ __device__ constexpr size_t target_cube_lds(int n) {
 // per side first, one block of CUBE_NT threads each, then the cubes of four
 // grid points per side, one per wavefront in its own LDS slice.
 template <typename T>
-__global__ void __launch_bounds__(CUBE_NT) k_target(const TgtPlan* __restrict__ tgt, int nbig, int ntgt,
+__global__ void __launch_bounds__(CUBE_NT, sizeof(T) == 4 ? 6 : 2) k_target(const TgtPlan* __restrict__ tgt, int nbig, int ntgt,
                                                     const T* __restrict__ UTI,
                                                     const typename Cplx<T>::type* __restrict__ acc,
                                                     T* __restrict__ w, int wave_lds, int nb, int ncol,
@@ -1447,42 +1822,49 @@ __global__ void __launch_bounds__(CUBE_NT) k_target(const TgtPlan* __restrict__ 
    const int wave = threadIdx.x >> 6, i = nbig + (cb.b - nbig) * (CUBE_NT / 64) + wave;
    if (i >= ntgt) return;
    const TgtPlan d = tgt[i];
-   target_body<4, T>(d, UTI, acc, w, smem + (size_t)wave * wave_lds, WaveGroup{(int)(threadIdx.x & 63)});
+   target4<T, 1>(d, UTI, acc, 0, w, 0, 1, smem + (size_t)wave * wave_lds, threadIdx.x & 63);
 }
 
-// k_target for TGT_NC columns per block or wavefront (column-batched
-// applies), with the extra grid values of each column in the LDS slice.
+// Column batches: TGT_NC columns of a cube of four grid points per side per
+// wavefront, which share each read of UTI.
 constexpr int TGT_NC = 4;
 template <typename T>
-__global__ void __launch_bounds__(CUBE_NT) k_target_mc(const TgtPlan* __restrict__ tgt, int nbig, int ntgt,
+__global__ void __launch_bounds__(CUBE_NT, sizeof(T) == 4 ? 6 : 4)
+    k_target4_mc(const TgtPlan* __restrict__ tgt, int ntgt, const T* __restrict__ UTI,
+                 const typename Cplx<T>::type* __restrict__ acc, T* __restrict__ w, int wave_lds, int nb, int ncol,
+                 long long cs_acc, long long cs_w) {
+   extern __shared__ __align__(16) unsigned char smem[];
+   const ColBlk cb = col_block((ncol + TGT_NC - 1) / TGT_NC);
+   const int wave = threadIdx.x >> 6, i = cb.b * (CUBE_NT / 64) + wave, c0 = cb.c * TGT_NC;
+   if (cb.b >= nb || i >= ntgt) return;
+   const TgtPlan d = tgt[i];
+   target4<T, TGT_NC>(d, UTI, acc + c0 * cs_acc, cs_acc, w + c0 * cs_w, cs_w, min(TGT_NC, ncol - c0),
+                      smem + (size_t)wave * wave_lds, threadIdx.x & 63);
+}
+
+// The other cubes, one block each, TGT_NC columns per block (FP64), with the
+// extra grid values of each column in LDS.
+template <typename T>
+__global__ void __launch_bounds__(CUBE_NT) k_target_mc(const TgtPlan* __restrict__ tgt, int ntgt,
                                                        const T* __restrict__ UTI,
                                                        const typename Cplx<T>::type* __restrict__ acc,
-                                                       T* __restrict__ w, int wave_lds, int nb, int ncol,
-                                                       long long cs_acc, long long cs_w) {
+                                                       T* __restrict__ w, int ncol, long long cs_acc,
+                                                       long long cs_w) {
    extern __shared__ __align__(16) unsigned char smem[];
-   const int ngrp = (ncol + TGT_NC - 1) / TGT_NC;
-   const ColBlk cb = col_block(ngrp);
-   if (cb.b >= nb) return;
+   const ColBlk cb = col_block((ncol + TGT_NC - 1) / TGT_NC);
+   if (cb.b >= ntgt) return;
    const int c0 = cb.c * TGT_NC, nc = min(TGT_NC, ncol - c0);
-   if (cb.b < nbig) {
-      const TgtPlan d = tgt[cb.b];
-      const BlockGroup gr = block_group();
-      switch (d.n) {
-         case 3: target_body_mc<3, T, TGT_NC>(d, UTI, acc, cs_acc, w, cs_w, c0, nc, smem, gr); break;
-         case 5: target_body_mc<5, T, TGT_NC>(d, UTI, acc, cs_acc, w, cs_w, c0, nc, smem, gr); break;
-         case 6: target_body_mc<6, T, TGT_NC>(d, UTI, acc, cs_acc, w, cs_w, c0, nc, smem, gr); break;
-         case 7: target_body_mc<7, T, TGT_NC>(d, UTI, acc, cs_acc, w, cs_w, c0, nc, smem, gr); break;
-         case 8: target_body_mc<8, T, TGT_NC>(d, UTI, acc, cs_acc, w, cs_w, c0, nc, smem, gr); break;
-         case 9: target_body_mc<9, T, TGT_NC>(d, UTI, acc, cs_acc, w, cs_w, c0, nc, smem, gr); break;
-         default: break;
-      }
-      return;
+   const TgtPlan d = tgt[cb.b];
+   const BlockGroup gr = block_group();
+   switch (d.n) {
+      case 3: target_body_mc<3, T, TGT_NC>(d, UTI, acc, cs_acc, w, cs_w, c0, nc, smem, gr); break;
+      case 5: target_body_mc<5, T, TGT_NC>(d, UTI, acc, cs_acc, w, cs_w, c0, nc, smem, gr); break;
+      case 6: target_body_mc<6, T, TGT_NC>(d, UTI, acc, cs_acc, w, cs_w, c0, nc, smem, gr); break;
+      case 7: target_body_mc<7, T, TGT_NC>(d, UTI, acc, cs_acc, w, cs_w, c0, nc, smem, gr); break;
+      case 8: target_body_mc<8, T, TGT_NC>(d, UTI, acc, cs_acc, w, cs_w, c0, nc, smem, gr); break;
+      case 9: target_body_mc<9, T, TGT_NC>(d, UTI, acc, cs_acc, w, cs_w, c0, nc, smem, gr); break;
+      default: break;
    }
-   const int wave = threadIdx.x >> 6, i = nbig + (cb.b - nbig) * (CUBE_NT / 64) + wave;
-   if (i >= ntgt) return;
-   const TgtPlan d = tgt[i];
-   target_body_mc<4, T, TGT_NC>(d, UTI, acc, cs_acc, w, cs_w, c0, nc, smem + (size_t)wave * wave_lds,
-                                WaveGroup{(int)(threadIdx.x & 63)});
 }
 
 // Leaf output: y = D_s xs + D_d xd (interleaved 2p x m block) + sum over the
@@ -1939,7 +2321,7 @@ void launch_apply_stage(int stage, const ApplyArgs& a, hipStream_t s) {
          break;
       }
       case 1: {
-         const int wl = (int)((source_cube_lds<T>(4, a.maxr_src, 64) + 15) / 16 * 16);
+         const int wl = (int)source4_lds<T>(a.maxr_src, 1);
          size_t lds = (size_t)(CUBE_NT / 64) * wl;
          for (int n = 3; n <= a.max_n; n++)
             if (n != 4) lds = std::max(lds, source_cube_lds<T>(n, a.maxr_src, CUBE_NT));
@@ -1952,13 +2334,26 @@ void launch_apply_stage(int stage, const ApplyArgs& a, hipStream_t s) {
                                            hipFuncAttributeMaxDynamicSharedMemorySize, 163840));
             FSVD_CHECK(hipFuncSetAttribute((const void*)k_source<T, true, 1>,
                                            hipFuncAttributeMaxDynamicSharedMemorySize, 163840));
+            FSVD_CHECK(hipFuncSetAttribute((const void*)k_source_mc<T>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                           163840));
          });
-         const int nb = a.nsrc_big + (a.nsrc - a.nsrc_big + CUBE_NT / 64 - 1) / (CUBE_NT / 64);
+         // batches: the wavefronts' cubes by groups of columns, unless their
+         // ranks are too large for the groups' LDS
+         const size_t wlm = source4_lds<T>(a.maxr_src, SRC_NC<T>);
+         const bool mc = a.ncol > 1 && (CUBE_NT / 64) * wlm <= 163840;
+         const int nsrc = mc ? a.nsrc_big : a.nsrc;
+         const int nb = a.nsrc_big + (nsrc - a.nsrc_big + CUBE_NT / 64 - 1) / (CUBE_NT / 64);
          if (nb) {
             auto kern = a.layers == 1 ? k_source<T, true, 1> : (a.ncol == 1 ? k_source<T, true, 2> : k_source<T, false, 2>);
-            hipLaunchKernelGGL(kern, dim3(col_grid(nb, a.ncol)), dim3(CUBE_NT), lds, s, a.src, a.nsrc_big, a.nsrc,
+            hipLaunchKernelGGL(kern, dim3(col_grid(nb, a.ncol)), dim3(CUBE_NT), lds, s, a.src, a.nsrc_big, nsrc,
                                (const T*)a.tpart, (const T*)a.PV, (C2*)a.spec, wl, nb, a.ncol, a.cs_tpart,
                                a.cs_spec);
+         }
+         if (mc && a.nsrc > a.nsrc_big) {
+            const int n4 = a.nsrc - a.nsrc_big, nb4 = (n4 + CUBE_NT / 64 - 1) / (CUBE_NT / 64);
+            hipLaunchKernelGGL((k_source_mc<T>), dim3(col_grid(nb4, (a.ncol + SRC_NC<T> - 1) / SRC_NC<T>)), dim3(CUBE_NT),
+                               (CUBE_NT / 64) * wlm, s, a.src + a.nsrc_big, n4, (const T*)a.tpart, (const T*)a.PV,
+                               (C2*)a.spec, (int)wlm, nb4, a.ncol, a.cs_tpart, a.cs_spec);
          }
          break;
       }
@@ -1992,43 +2387,47 @@ void launch_apply_stage(int stage, const ApplyArgs& a, hipStream_t s) {
          break;
       }
       case 3: {
-         const int wl = (int)((target_cube_lds<T>(4) + 15) / 16 * 16);
-         size_t lds = (size_t)(CUBE_NT / 64) * wl;
+         const int wl = (int)target4_lds<T>(1), wlm = (int)target4_lds<T>(TGT_NC);
+         size_t lds = (size_t)(CUBE_NT / 64) * wl, lmc = 0;
          for (int n = 3; n <= a.max_n; n++)
-            if (n != 4) lds = std::max(lds, target_cube_lds<T>(n));
+            if (n != 4) {
+               lds = std::max(lds, target_cube_lds<T>(n));
+               lmc = std::max(lmc, target_cube_lds<T>(n) + sizeof(T) * (size_t)(TGT_NC - 1) * n * n * n);
+            }
          check_lds(lds);
          static std::once_flag attr;   // large n needs more than the default dynamic LDS
          std::call_once(attr, [] {
             FSVD_CHECK(hipFuncSetAttribute((const void*)k_target<T>, hipFuncAttributeMaxDynamicSharedMemorySize,
                                            163840));
-         });
-         const int nb = a.ntgt_big + (a.ntgt - a.ntgt_big + CUBE_NT / 64 - 1) / (CUBE_NT / 64);
-         if (nb && (a.ncol == 1 || sizeof(T) == 4)) {
-            // FP32 batches run one block copy per column: the FP32 UTI rows
-            // are cheap to re-read from L2, and the transforms run in
-            // parallel (0.033 against 0.042 ms per column for four columns
-            // per block on the 100k-panel globule)
-            hipLaunchKernelGGL((k_target<T>), dim3(col_grid(nb, a.ncol)), dim3(CUBE_NT), lds, s, a.tgt, a.ntgt_big,
-                               a.ntgt, (const T*)a.UTI, (const C2*)a.acc, (T*)a.w, wl, nb, a.ncol, a.cs_acc, a.cs_w);
-         } else if (nb) {
-            // FP64: TGT_NC columns per block, their grid values beside the
-            // transform buffers (0.052 against 0.063 ms per column)
-            const size_t extra4 = sizeof(T) * (size_t)(TGT_NC - 1) * 64;
-            const int wlm = (int)((target_cube_lds<T>(4) + extra4 + 15) / 16 * 16);
-            size_t lmc = (size_t)(CUBE_NT / 64) * wlm;
-            for (int n = 3; n <= a.max_n; n++)
-               if (n != 4)
-                  lmc = std::max(lmc, target_cube_lds<T>(n) + sizeof(T) * (size_t)(TGT_NC - 1) * n * n * n);
-            check_lds(lmc);
-            static std::once_flag attr_mc;
-            std::call_once(attr_mc, [] {
-               FSVD_CHECK(hipFuncSetAttribute((const void*)k_target_mc<T>,
+            FSVD_CHECK(hipFuncSetAttribute((const void*)k_target4_mc<T>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                           163840));
+            if (sizeof(T) == 8)
+               FSVD_CHECK(hipFuncSetAttribute((const void*)k_target_mc<double>,
                                               hipFuncAttributeMaxDynamicSharedMemorySize, 163840));
-            });
-            const int ngrp = (a.ncol + TGT_NC - 1) / TGT_NC;
-            hipLaunchKernelGGL((k_target_mc<T>), dim3(col_grid(nb, ngrp)), dim3(CUBE_NT), lmc, s, a.tgt, a.ntgt_big,
-                               a.ntgt, (const T*)a.UTI, (const C2*)a.acc, (T*)a.w, wlm, nb, a.ncol, a.cs_acc,
-                               a.cs_w);
+         });
+         // Batches: the wavefronts' cubes by groups of TGT_NC columns.  The
+         // large cubes, with one block each: in groups for FP64 (0.052 against
+         // 0.063 ms per column on the 100k-panel globule), a block per column
+         // for FP32 (0.033 against 0.042).
+         const bool mc = a.ncol > 1, bigmc = mc && sizeof(T) == 8;
+         const int ngrp = (a.ncol + TGT_NC - 1) / TGT_NC, n4 = a.ntgt - a.ntgt_big;
+         if constexpr (sizeof(T) == 8) {
+            if (bigmc && a.ntgt_big) {
+               check_lds(lmc);
+               hipLaunchKernelGGL((k_target_mc<T>), dim3(col_grid(a.ntgt_big, ngrp)), dim3(CUBE_NT), lmc, s, a.tgt,
+                                  a.ntgt_big, (const T*)a.UTI, (const C2*)a.acc, (T*)a.w, a.ncol, a.cs_acc, a.cs_w);
+            }
+         }
+         const int nt = mc ? (bigmc ? 0 : a.ntgt_big) : a.ntgt;
+         const int nb = nt ? a.ntgt_big + (nt - a.ntgt_big + CUBE_NT / 64 - 1) / (CUBE_NT / 64) : 0;
+         if (nb)
+            hipLaunchKernelGGL((k_target<T>), dim3(col_grid(nb, a.ncol)), dim3(CUBE_NT), lds, s, a.tgt, a.ntgt_big,
+                               nt, (const T*)a.UTI, (const C2*)a.acc, (T*)a.w, wl, nb, a.ncol, a.cs_acc, a.cs_w);
+         if (mc && n4 > 0) {
+            const int nb4 = (n4 + CUBE_NT / 64 - 1) / (CUBE_NT / 64);
+            hipLaunchKernelGGL((k_target4_mc<T>), dim3(col_grid(nb4, ngrp)), dim3(CUBE_NT), (CUBE_NT / 64) * wlm, s,
+                               a.tgt + a.ntgt_big, n4, (const T*)a.UTI, (const C2*)a.acc, (T*)a.w, wlm, nb4, a.ncol,
+                               a.cs_acc, a.cs_w);
          }
          break;
       }
