@@ -38,8 +38,7 @@ constexpr int ROUND_BLOCKS = 1024; // 4 waves for each of 1024 SIMDs
 // --- sums over panels: charges on lanes -------------------------------------
 // part[(sp * ncol + col) * nq + j], block (group of 64 charges, part sp)
 
-// Coulomb: sum_e lam[out[e]] / |c_e - x_j|
-// Integrals: sum_e (a_e slp - b_e dlp) - (self ? 4 pi b_e : 0) with Laplace
+// Potentials: sum_e (a_e slp - b_e dlp) - (self ? 4 pi b_e : 0) with Laplace
 // integrals of panel pidx[e] at the charge (direct branch of
 // SurfaceOperator_calculateReactionPotentials, SurfaceOperator.c:364-396).
 // For own panels a = sol[dphi], b = sol[phi], self check on; for child
@@ -88,6 +87,7 @@ __global__ void __launch_bounds__(256) k_potentials(int ne, int nq, int ncol, in
    }
 }
 
+// Transposed right-hand side: sum_e lam[out[e]] / |c_e - x_j|
 __global__ void __launch_bounds__(256) k_rhs_t(int ne, int nq, int ng, int per, const double* __restrict__ cent,
                                                const int* __restrict__ out, const double* __restrict__ lam,
                                                const double* __restrict__ qpos, double* __restrict__ part) {

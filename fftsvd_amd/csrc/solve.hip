@@ -1,6 +1,4 @@
-// Region-operator glue, block preconditioner, Krylov vector kernels, the
-// charge right-hand side and the reaction potentials at the charges.  All
-// FP64.
+// Region-operator glue, block preconditioner and Krylov vector kernels.
 #include <hip/hip_runtime.h>
 
 #include <type_traits>
