@@ -37,18 +37,19 @@ struct GemmDesc {
 };
 
 // Pivoted-MGS basis problem: A (rows x cols, column-major, column j at
-// a_off + j*lda, lda even and a_off even so that columns start 16-byte
-// aligned; modified in place) -> rank (rank_slot) and the first `rank`
+// a_off + j*rows, modified in place) -> rank (rank_slot) and the first `rank`
 // orthonormal pivot columns at q_off (column k at q_off + k*rows).
-// seg, nb, ws_off are set by the host scheduler (run_mgs).
+// MGS_SLACK readable values follow the last matrix.  The rest is set by the
+// host scheduler (run_mgs).
+constexpr int MGS_SLACK = 4 * 64;
 struct MgsDesc {
-   int rows, cols, lda;
+   int rows, cols;
    long long a_off;
    long long q_off;
    int rank_slot;
-   int seg;             // register kernel: lanes per column pair
+   int seg;             // lanes that share a column's sums
    int nb;              // blocked kernel: steps per block
-   long long ws_off;    // blocked kernel: its arrays in the global scratch (when not in LDS)
+   long long ws_off;    // k_mgs_long: its arrays in the scratch
 };
 
 // Near-field leaf: rows q0..q0+p-1 (tree-order points), m columns listed at

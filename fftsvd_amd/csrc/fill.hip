@@ -113,23 +113,35 @@ __global__ void __launch_bounds__(256) k_gemm_batched(const GemmDesc* __restrict
 }
 
 // ---------------------------------------------------------------------------
-// Column bases by pivoted MGS with the rank cut ||col|| < eps*||A||_F
-// (reference Matrix_columnbasis_pivotedmgs, Matrix.c:215-307): at step k the
-// remaining column of largest norm (ties to the lowest current position,
-// positions k and the pivot's exchanged, as the reference exchanges columns)
-// becomes q_k and is projected out of the rest.  One workgroup runs one
-// problem from its first to its last step, so a batch is a launch or two
-// instead of a pair of launches per step:
-//   k_mgs_reg  the matrix in registers (at most 16 rows x 64 lanes by 2 x
-//              1024/lanes columns: the leaf cubes and most of the next level)
-//   k_mgs_blk  larger matrices, read from L2 once per step and written once
-//              per block of steps
-// Kernel time of one operator pair's bases (MI355X), against one launch per
-// pivot step with the matrices read and written in each: 31 000 panels
-// 61 -> 37 ms in 60 launches instead of 1700, 100 000 panels 228 -> 81 ms.
+// Column bases by pivoted MGS with two re-orthogonalisations and the rank cut
+// ||col|| < eps*||A||_F (reference Matrix_columnbasis_pivotedmgs,
+// Matrix.c:215-307): at step k the remaining column of largest norm (ties to
+// the lowest current position, positions k and the pivot's exchanged, as the
+// reference exchanges columns) becomes q_k = a / |a|, and the others have it
+// taken out twice, a -= (q . a) q, and their norms formed afresh.
+//
+// The order of every sum is fixed by rows and cols alone (mgs_sum_lanes), so
+// that a basis does not depend on the kernel that makes it: one lane, first
+// row to last, where the matrix fits 96 KB; else the rows sl, sl + S, sl + 2S,
+// ... per lane sl of S, the lanes' sums then added pairwise, lanes S/2 apart
+// first.  Bases of the same span with other rounding move an FP64 product by
+// up to 1e-13 of its norm: directions that the steps leave small are their
+// rounding errors' size.
+//
+// One workgroup runs a problem from its first to its last step, so a batch is
+// a dozen launches at most:
+//   k_mgs_cols  one lane per column, columns in registers and LDS
+//   k_mgs_reg   S lanes per two columns, all in registers
+//   k_mgs_blk   larger ones, read from L2 once per step
+//   k_mgs_long  the rest (more than 6144 rows)
+// Against two launches per step over all problems, each reading and writing
+// every matrix: one operator pair's bases take 130 ms of kernel time instead of
+// 212 at 100 000 panels (130 launches instead of 2180), 63 instead of 59 at
+// 31 000; the operators are there after 140 and 64 ms instead of 206 and 105,
+// with the kept device memory.
 
-// Value of another lane of the row by DPP (quad permutations, half-row and
-// row mirrors): VALU moves, without the LDS round trip of a shuffle.
+// Value of another lane of the row by DPP (quad permutations, half-row mirror,
+// row rotation): VALU moves, without the LDS round trip of a shuffle.
 template <int CTRL>
 __device__ __forceinline__ int dpp_i(int v) {
    return __builtin_amdgcn_update_dpp(0, v, CTRL, 0xf, 0xf, true);
@@ -138,18 +150,17 @@ template <int CTRL>
 __device__ __forceinline__ double dpp_d(double v) {
    return __hiloint2double(dpp_i<CTRL>(__double2hiint(v)), dpp_i<CTRL>(__double2loint(v)));
 }
-constexpr int DPP_XOR1 = 0xB1, DPP_XOR2 = 0x4E, DPP_HALF_MIRROR = 0x141, DPP_MIRROR = 0x140;
+constexpr int DPP_XOR1 = 0xB1, DPP_XOR2 = 0x4E, DPP_XOR3 = 0x1B, DPP_XOR7 = 0x141, DPP_XOR8 = 0x128;
 
-// Sum over the S lanes (a power of two) of the lane's aligned segment, the
-// same in all of them.  The mirrors pair lanes whose quads (half rows)
-// already hold equal sums, so they act as exchanges with the lane 4 (8) away.
+// Sum over the S lanes (a power of two) of the lane's aligned segment, lanes
+// S/2 apart first; the same in all of them.
 __device__ __forceinline__ double seg_sum(double v, int S) {
-   if (S > 1) v += dpp_d<DPP_XOR1>(v);
-   if (S > 2) v += dpp_d<DPP_XOR2>(v);
-   if (S > 4) v += dpp_d<DPP_HALF_MIRROR>(v);
-   if (S > 8) v += dpp_d<DPP_MIRROR>(v);
-   if (S > 16) v += __shfl_xor(v, 16, 64);
    if (S > 32) v += __shfl_xor(v, 32, 64);
+   if (S > 16) v += __shfl_xor(v, 16, 64);
+   if (S > 8) v += dpp_d<DPP_XOR8>(v);
+   if (S > 4) v += dpp_d<DPP_XOR3>(dpp_d<DPP_XOR7>(v));
+   if (S > 2) v += dpp_d<DPP_XOR2>(v);
+   if (S > 1) v += dpp_d<DPP_XOR1>(v);
    return v;
 }
 // Largest value over the wave (NaN ignored) and, among the lanes that hold
@@ -157,314 +168,463 @@ __device__ __forceinline__ double seg_sum(double v, int S) {
 __device__ __forceinline__ double wave_max(double v) {
    v = fmax(v, dpp_d<DPP_XOR1>(v));
    v = fmax(v, dpp_d<DPP_XOR2>(v));
-   v = fmax(v, dpp_d<DPP_HALF_MIRROR>(v));
-   v = fmax(v, dpp_d<DPP_MIRROR>(v));
+   v = fmax(v, dpp_d<DPP_XOR7>(v));
+   v = fmax(v, dpp_d<DPP_XOR8>(v));
    v = fmax(v, __shfl_xor(v, 16, 64));
    return fmax(v, __shfl_xor(v, 32, 64));
 }
 __device__ __forceinline__ int wave_min(int v) {
    v = min(v, dpp_i<DPP_XOR1>(v));
    v = min(v, dpp_i<DPP_XOR2>(v));
-   v = min(v, dpp_i<DPP_HALF_MIRROR>(v));
-   v = min(v, dpp_i<DPP_MIRROR>(v));
+   v = min(v, dpp_i<DPP_XOR7>(v));
+   v = min(v, dpp_i<DPP_XOR8>(v));
    v = min(v, __shfl_xor(v, 16, 64));
    return min(v, __shfl_xor(v, 32, 64));
 }
 
-// Sum over the block, the same in every thread; red holds one value per
-// wave.  A barrier separates consecutive uses of red.
-__device__ __forceinline__ double block_total(double v, double* red, int nw) {
-   v = seg_sum(v, 64);
-   if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
+// The pivot of a step: largest norm (0 if none is above it) and its position
+// over the block, from each thread's candidate.  wv, wp: a value per wave,
+// free for reuse after the caller's next barrier.
+__device__ __forceinline__ void block_pivot(double bv, int bp, int nw, double* wv, int* wp, double& mx, int& best) {
+   mx = wave_max(bv);
+   best = wave_min(bv == mx ? bp : 0x7fffffff);
+   if ((threadIdx.x & 63) == 0) {
+      wv[threadIdx.x >> 6] = mx;
+      wp[threadIdx.x >> 6] = best;
+   }
    __syncthreads();
-   double t = 0.0;
-   for (int w = 0; w < nw; w++) t += red[w];
-   __syncthreads();
-   return t;
+   mx = wv[0];
+   best = wp[0];
+   for (int w = 1; w < nw; w++) {
+      const double ov = wv[w];
+      const int op = wp[w];
+      if (ov > mx || (ov == mx && op < best)) {
+         mx = ov;
+         best = op;
+      }
+   }
 }
 
-// Register kernel.  S = seg lanes share two columns (j = g and g + NT/S of
-// lane group g), 16 rows of each per lane: row pairs 2 (sl + S u), u < 8, so
-// that the pivot vector is read from LDS in conflict-free 16-byte pieces,
-// once per step, into registers.  Each step makes the two projections
-// a -= (q . a) q of the reference's re-orthogonalising MGS and the fresh
-// squared norm.  FP64 rate and the two barriers of a step bound it; the
-// matrix is read from HBM once.  (The 16 300 leaf problems of a 100 000-panel
-// tree took 10 ms with the matrix in LDS, a thread per column: 96 KB of LDS
-// left one workgroup per CU.)
+// Frobenius norm from the squared column norms n2 (LDS), in every lane: 256
+// sums over the columns 256 apart, added pairwise, 128 apart first.
+__device__ __forceinline__ double mgs_frobenius(const double* n2, int cols) {
+   double p[4];
+#pragma unroll
+   for (int q = 0; q < 4; q++) {
+      p[q] = 0.0;
+      for (int j = (threadIdx.x & 63) + 64 * q; j < cols; j += 256) p[q] += n2[j];
+   }
+   return sqrt(seg_sum((p[0] + p[2]) + (p[1] + p[3]), 64));
+}
+
+// One lane per column: rows 0 .. NR - 1 in registers, the others in LDS (rem,
+// row-major).  Bound by the FP64 rate, the latency of the sums' chains where
+// few waves share a CU, and three barriers a step.
+constexpr int mgs_cols_threads(int NR) { return NR == 32 ? 1024 : (NR == 64 ? 512 : 256); }
+__host__ __device__ inline size_t mgs_cols_bytes(int rows, int cols, int NR) {
+   return sizeof(double) * ((size_t)(rows > NR ? rows : NR) + (size_t)cols * (rows > NR ? rows - NR : 0));
+}
+template <int NR>
+__global__ void __launch_bounds__(mgs_cols_threads(NR))
+    k_mgs_cols(const MgsDesc* __restrict__ descs, const int* __restrict__ list, const double* __restrict__ Abuf,
+               double* __restrict__ Qbuf, int* __restrict__ ranks, double eps) {
+   constexpr int NT = mgs_cols_threads(NR), G = 8;
+   extern __shared__ __align__(16) unsigned char sm[];
+   __shared__ double n2[NT];
+   __shared__ double wv[NT / 64];
+   __shared__ int wp[NT / 64];
+   const MgsDesc d = descs[list[blockIdx.x]];
+   const int rows = d.rows, cols = d.cols, tid = threadIdx.x, nw = (int)blockDim.x >> 6;
+   double* qs = (double*)sm;                      // rows, zeros up to NR
+   double* rem = qs + max(rows, NR) + tid;        // (rows - NR) x cols
+   const bool mine = tid < cols, busy = (tid & ~63) < cols;   // busy: a wave with columns
+   const double* a = Abuf + d.a_off + (long long)(mine ? tid : 0) * rows;
+   double v[NR];
+   double sq = 0.0;
+#pragma unroll
+   for (int t = 0; t < NR; t++) v[t] = t < rows && mine ? a[t < rows ? t : 0] : 0.0;
+#pragma unroll
+   for (int t = 0; t < NR; t++) sq = fma(v[t], v[t], sq);
+   if (mine)
+      for (int t = NR; t < rows; t++) {
+         const double x = a[t];
+         rem[(size_t)(t - NR) * cols] = x;
+         sq = fma(x, x, sq);
+      }
+   n2[tid] = sq;
+   for (int t = rows + tid; t < NR; t += (int)blockDim.x) qs[t] = 0.0;
+   __syncthreads();
+   const double cut = eps * mgs_frobenius(n2, cols);
+   double nrm = sqrt(sq);
+   int pos = mine ? tid : -1;   // the column's current position; -1: taken or none
+   const int kmax = min(rows, cols);
+   int k = 0;
+   for (; k < kmax; k++) {
+      double mx;
+      int best;
+      const bool on = pos >= k && nrm >= 0.0;
+      block_pivot(on ? nrm : 0.0, on ? pos : 0x7fffffff, nw, wv, wp, mx, best);
+      if (!(mx > 0.0)) best = k;
+      if (k >= 1 && mx < cut) break;   // uniform over the block
+      if (pos == best) {
+#pragma unroll
+         for (int t = 0; t < NR; t++)
+            if (t < rows) qs[t] = v[t];
+         for (int t = NR; t < rows; t++) qs[t] = rem[(size_t)(t - NR) * cols];
+         pos = -1;
+      } else if (pos == k) {
+         pos = best;
+      }
+      __syncthreads();
+      for (int t = tid; t < rows; t += (int)blockDim.x) {
+         const double x = qs[t] / mx;
+         qs[t] = x;
+         Qbuf[d.q_off + (long long)k * rows + t] = x;
+      }
+      __syncthreads();
+      if (busy) {
+         // r1 = q.a; a -= r1 q, r2 = q.a; a -= r2 q, |a|^2
+         double r1 = 0.0, r2 = 0.0;
+         sq = 0.0;
+#pragma unroll
+         for (int g = 0; g < NR; g += G)
+            if (g < rows)
+#pragma unroll
+               for (int t = g; t < g + G; t++) r1 = fma(qs[t], v[t], r1);
+         if (mine)
+            for (int t = NR; t < rows; t++) r1 = fma(qs[t], rem[(size_t)(t - NR) * cols], r1);
+#pragma unroll
+         for (int g = 0; g < NR; g += G)
+            if (g < rows)
+#pragma unroll
+               for (int t = g; t < g + G; t++) {
+                  const double q = qs[t];
+                  v[t] = fma(-q, r1, v[t]);
+                  r2 = fma(q, v[t], r2);
+               }
+         if (mine)
+            for (int t = NR; t < rows; t++) {
+               const double q = qs[t], x = fma(-q, r1, rem[(size_t)(t - NR) * cols]);
+               rem[(size_t)(t - NR) * cols] = x;
+               r2 = fma(q, x, r2);
+            }
+#pragma unroll
+         for (int g = 0; g < NR; g += G)
+            if (g < rows)
+#pragma unroll
+               for (int t = g; t < g + G; t++) {
+                  v[t] = fma(-qs[t], r2, v[t]);
+                  sq = fma(v[t], v[t], sq);
+               }
+         if (mine)
+            for (int t = NR; t < rows; t++) {
+               const double x = fma(-qs[t], r2, rem[(size_t)(t - NR) * cols]);
+               rem[(size_t)(t - NR) * cols] = x;
+               sq = fma(x, x, sq);
+            }
+         nrm = sqrt(sq);
+      }
+   }
+   if (tid == 0) ranks[d.rank_slot] = k;
+}
+
+// The lane's rows i = sl, sl + S, ... of a column, at most NR: four at a time
+// while there are any (what they read past the column's end, of the next
+// columns or the MGS_SLACK values after the last, mgs_mask makes zeros), the
+// others zero.  One lane offset for all rows, so that their addresses cost no
+// registers.
+template <int NR>
+__device__ __forceinline__ void mgs_load(double (&x)[NR], const double* A, unsigned at, int rows, int S) {
+#pragma unroll
+   for (int t0 = 0; t0 < NR; t0 += 4)
+      if (S * t0 < rows) {
+#pragma unroll
+         for (int t = t0; t < t0 + 4; t++) x[t] = (A + S * t)[at];
+      } else {
+#pragma unroll
+         for (int t = t0; t < t0 + 4; t++) x[t] = 0.0;
+      }
+}
+template <int NR>
+__device__ __forceinline__ void mgs_mask(double (&x)[NR], int rows, int S, int sl) {
+#pragma unroll
+   for (int t0 = 0; t0 < NR; t0 += 4)
+      if (S * t0 < rows && S * (t0 + 4) > rows)
+#pragma unroll
+         for (int t = t0; t < t0 + 4; t++) x[t] = sl < rows - S * t ? x[t] : 0.0;
+}
+
+// S lanes per two columns (j = g and g + NT/S of lane group g), at most 16
+// rows of each per lane.  Bound by the FP64 rate and three barriers a step;
+// the matrix is read from HBM once.
 constexpr int MGS_NR = 16;
 template <int NT>
 __global__ void __launch_bounds__(NT) k_mgs_reg(const MgsDesc* __restrict__ descs, const int* __restrict__ list,
                                                 const double* __restrict__ Abuf, double* __restrict__ Qbuf,
                                                 int* __restrict__ ranks, double eps) {
-   constexpr int NW = NT / 64, NP = MGS_NR / 2;
-   __shared__ __align__(16) double qs[MGS_NR * 64];
-   __shared__ double wv[NW];
-   __shared__ int wp[NW];
+   __shared__ double qs[MGS_NR * 64];
+   __shared__ double n2[NT / 2];   // S >= 4
+   __shared__ double wv[NT / 64];
+   __shared__ int wp[NT / 64];
    const MgsDesc d = descs[list[blockIdx.x]];
-   const int rows = d.rows, cols = d.cols, S = d.seg, tid = threadIdx.x, wave = tid >> 6;
+   const int rows = d.rows, cols = d.cols, S = d.seg, tid = threadIdx.x;
    const int g = tid / S, sl = tid - g * S, G = NT / S;
    double v[2][MGS_NR];
-   double n2[2];
-   int pos[2];   // the column's current position; INT_MAX: none, -1: taken
+   double nrm[2];
+   int pos[2];   // the column's current position; -1: taken or none
 #pragma unroll
    for (int c = 0; c < 2; c++) {
       const int j = g + c * G;
-      const double* a = Abuf + d.a_off + (long long)(j < cols ? j : 0) * d.lda;
-      pos[c] = j < cols ? j : 0x7fffffff;
+      pos[c] = j < cols ? j : -1;
       double s = 0.0;
+      mgs_load(v[c], Abuf + d.a_off, (unsigned)((j < cols ? j : 0) * rows + sl), rows, S);
+      mgs_mask(v[c], rows, S, sl);
 #pragma unroll
-      for (int u = 0; u < NP; u++) {
-         const int i = 2 * (sl + S * u);
-         // the even column stride makes row i + 1 readable whenever row i is
-         const double2 x = *(const double2*)(a + (i < rows ? i : 0));
-         v[c][2 * u] = j < cols && i < rows ? x.x : 0.0;
-         v[c][2 * u + 1] = j < cols && i + 1 < rows ? x.y : 0.0;
-      }
+      for (int t = 0; t < MGS_NR; t++) v[c][t] = j < cols ? v[c][t] : 0.0;
 #pragma unroll
       for (int t = 0; t < MGS_NR; t++) s = fma(v[c][t], v[c][t], s);
-      n2[c] = seg_sum(s, S);
+      s = seg_sum(s, S);
+      if (sl == 0) n2[j] = s;
+      nrm[c] = sqrt(s);
    }
-   const double fro = sqrt(block_total(sl == 0 ? n2[0] + n2[1] : 0.0, wv, NW));
+   for (int i = rows + tid; i < MGS_NR * S; i += NT) qs[i] = 0.0;   // past the last row
+   __syncthreads();
+   const double cut = eps * mgs_frobenius(n2, cols);
    const int kmax = min(rows, cols);
    int k = 0;
    for (; k < kmax; k++) {
-      double bv = 0.0;
-      int bp = 0x7fffffff;
+      double bv = 0.0, mx;
+      int bp = 0x7fffffff, best;
 #pragma unroll
       for (int c = 0; c < 2; c++)
-         if (pos[c] >= k && pos[c] != 0x7fffffff && (n2[c] > bv || (n2[c] == bv && pos[c] < bp))) {
-            bv = n2[c];
+         if (pos[c] >= k && (nrm[c] > bv || (nrm[c] == bv && pos[c] < bp))) {
+            bv = nrm[c];
             bp = pos[c];
          }
-      double mx = wave_max(bv);
-      int best = wave_min(bv == mx ? bp : 0x7fffffff);
-      if constexpr (NW > 1) {
-         if ((tid & 63) == 0) {
-            wv[wave] = mx;
-            wp[wave] = best;
-         }
-         __syncthreads();
-         mx = wv[0];
-         best = wp[0];
-#pragma unroll
-         for (int w = 1; w < NW; w++) {
-            const double ov = wv[w];
-            const int op = wp[w];
-            if (ov > mx || (ov == mx && op < best)) {
-               mx = ov;
-               best = op;
-            }
-         }
-      }
+      block_pivot(bv, bp, NT / 64, wv, wp, mx, best);
       if (!(mx > 0.0)) best = k;
-      const double nrm = sqrt(mx);
-      if (k >= 1 && nrm < eps * fro) break;
-      double* q = Qbuf + d.q_off + (long long)k * rows;
+      if (k >= 1 && mx < cut) break;   // uniform over the block
 #pragma unroll
       for (int c = 0; c < 2; c++) {
          if (pos[c] == best) {
 #pragma unroll
-            for (int u = 0; u < NP; u++) {
-               const int i = 2 * (sl + S * u);
-               const double x = v[c][2 * u] / nrm, y = v[c][2 * u + 1] / nrm;
-               *(double2*)(qs + i) = make_double2(x, y);
-               if (i < rows) q[i] = x;
-               if (i + 1 < rows) q[i + 1] = y;
-            }
+            for (int t = 0; t < MGS_NR; t++)
+               if (sl + S * t < rows) qs[sl + S * t] = v[c][t];
             pos[c] = -1;
          } else if (pos[c] == k) {
             pos[c] = best;
          }
       }
       __syncthreads();
-      double p[MGS_NR];
-#pragma unroll
-      for (int u = 0; u < NP; u++) {
-         const double2 x = *(const double2*)(qs + 2 * (sl + S * u));
-         p[2 * u] = x.x;
-         p[2 * u + 1] = x.y;
+      for (int i = tid; i < rows; i += NT) {
+         const double x = qs[i] / mx;
+         qs[i] = x;
+         Qbuf[d.q_off + (long long)k * rows + i] = x;
       }
+      __syncthreads();
+      double q[MGS_NR];
+#pragma unroll
+      for (int t = 0; t < MGS_NR; t++) q[t] = qs[sl + S * t];
 #pragma unroll
       for (int c = 0; c < 2; c++) {
+         double r1 = 0.0, r2 = 0.0, s = 0.0;
 #pragma unroll
-         for (int pass = 0; pass < 2; pass++) {
-            double r0 = 0.0, r1 = 0.0;
+         for (int t = 0; t < MGS_NR; t++) r1 = fma(q[t], v[c][t], r1);
+         r1 = seg_sum(r1, S);
 #pragma unroll
-            for (int t = 0; t < MGS_NR; t += 2) {
-               r0 = fma(p[t], v[c][t], r0);
-               r1 = fma(p[t + 1], v[c][t + 1], r1);
-            }
-            const double r = seg_sum(r0 + r1, S);
-#pragma unroll
-            for (int t = 0; t < MGS_NR; t++) v[c][t] = fma(-p[t], r, v[c][t]);
+         for (int t = 0; t < MGS_NR; t++) {
+            v[c][t] = fma(-q[t], r1, v[c][t]);
+            r2 = fma(q[t], v[c][t], r2);
          }
-         double s0 = 0.0, s1 = 0.0;
+         r2 = seg_sum(r2, S);
 #pragma unroll
-         for (int t = 0; t < MGS_NR; t += 2) {
-            s0 = fma(v[c][t], v[c][t], s0);
-            s1 = fma(v[c][t + 1], v[c][t + 1], s1);
+         for (int t = 0; t < MGS_NR; t++) {
+            v[c][t] = fma(-q[t], r2, v[c][t]);
+            s = fma(v[c][t], v[c][t], s);
          }
-         n2[c] = seg_sum(s0 + s1, S);
+         nrm[c] = sqrt(seg_sum(s, S));
       }
-      // qs is rewritten after the next step's barrier (with one wave, by
-      // program order)
    }
    if (tid == 0) ranks[d.rank_slot] = k;
 }
 
-// Blocked kernel.  The columns stay as they were at the start of a block of
-// up to nb steps; a step reads them once for the products r_j = q_k . a_j,
-// kept in R, and takes r_j^2 off the squared norms; the block's end takes
-// the block's directions out of the columns and forms their squared norms
-// afresh.  A block also ends when the largest norm^2 has fallen by 1e-4, so
-// the running norms carry errors below 1e-12 relative to the largest, the
-// size of the columns' own rounding errors.  The pivot's vector takes the
-// block's products off its column and is then orthogonalised once more
-// against every earlier q (the reference re-orthogonalises against each q in
-// turn).  Columns whose norm^2 is below a quarter of the squared cut can
-// never be pivots and are no longer read.  The reads of the columns, from L2
-// and the Infinity Cache, and the latency of the step's phases bound it
-// (2986 x 160 at rank 70: 80 us a step), so 16 waves share a problem.
-// Arrays (LDS, or global scratch when GLB): v[rows rounded up to even],
-// R[nb * cols], n2[cols], h[min(rows, cols)], order[cols], act[cols].
-constexpr int MGS_BT = 1024;
-__host__ __device__ inline size_t mgs_blk_bytes(int rows, int cols, int nb) {
-   const int kmax = rows < cols ? rows : cols;
-   return sizeof(double) * ((size_t)cols * (nb + 1) + kmax + (rows + 1) / 2 * 2) + sizeof(int) * 2 * (size_t)cols + 16;
+// Larger matrices.  A stays in memory as it was at the start of a block of nb
+// steps; a step reads each column once, takes the block's earlier directions
+// out of it with the coefficients kept in R (the same operations on the same
+// values, so the same bits as a column written back every step), then does its
+// own two projections and the norm, all in registers; the block's last step
+// writes the columns back.  Up to NR rows a lane, 64 / S columns per wave.
+// Columns whose norm is below half of the cut can never be pivots and are no
+// longer read.  Bound by what one CU reads from L2 (about 60 GB/s) for long
+// columns, where few waves fit the registers, and by latency for short ones:
+// with PRE the next column is loaded during the work on one, the first of a
+// step during the choice of its pivot.  2986 x 160: 78 us a step; 3658 x 176:
+// 128; 662 of 316 x 176: 57 (nb = 2 or 4 the same; the registers that hold q
+// from one sum to the next cost more than its reads from LDS).
+// LDS: qs[nb * NR * S], R[nb * cols], n2[cols], order[cols], act[cols].
+__host__ __device__ inline size_t mgs_blk_bytes(int NRS, int cols, int nb) {
+   return sizeof(double) * (size_t)nb * NRS + sizeof(double2) * (size_t)nb * cols +
+          (sizeof(double) + 2 * sizeof(int)) * (size_t)cols;
 }
-template <bool GLB>
-__global__ void __launch_bounds__(MGS_BT) k_mgs_blk(const MgsDesc* __restrict__ descs, const int* __restrict__ list,
-                                                    double* __restrict__ Abuf, double* __restrict__ Qbuf,
-                                                    int* __restrict__ ranks, double eps,
-                                                    unsigned char* __restrict__ scratch) {
+template <int NR, int S, int NT, bool PRE>
+__global__ void __launch_bounds__(NT) k_mgs_blk(const MgsDesc* __restrict__ descs, const int* __restrict__ list,
+                                                double* __restrict__ Abuf, double* __restrict__ Qbuf,
+                                                int* __restrict__ ranks, double eps) {
    extern __shared__ __align__(16) unsigned char sm[];
-   __shared__ double red[MGS_BT / 64];
-   __shared__ int redi[MGS_BT / 64];
+   __shared__ double wv[NT / 64];
+   __shared__ int wp[NT / 64];
    __shared__ int s_nact;
-   constexpr int NW = MGS_BT / 64, U = 8;
+   constexpr int NW = NT / 64, G = NR > 32 ? 16 : 4;   // G: reads of q in flight, for few waves more
    const MgsDesc d = descs[list[blockIdx.x]];
-   const int m = d.rows, K = d.cols, NB = d.nb, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-   const int kmax = min(m, K), mpad = (m + 1) / 2 * 2;
-   const long long lda = d.lda;
+   constexpr int ldq = NR * S;
+   const int m = d.rows, K = d.cols, NB = d.nb;
+   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+   const int sub = lane / S, sl = lane - sub * S;
+   constexpr int CPW = 64 / S;   // columns per wave at a time
+   const int kmax = min(m, K);
    double* A = Abuf + d.a_off;
    double* Q = Qbuf + d.q_off;
-   double* v = (double*)(GLB ? scratch + d.ws_off : sm);   // first: 16-byte aligned
-   double* R = v + mpad;
-   double* n2 = R + (size_t)NB * K;
-   double* h = n2 + K;
-   int* order = (int*)(h + kmax);
+   double* qs = (double*)sm;
+   double2* R = (double2*)(qs + NB * ldq);
+   double* n2 = (double*)(R + NB * K);
+   int* order = (int*)(n2 + K);
    int* act = order + K;
-   // lanes per column: whole waves for long columns, parts of one for short
-   const int S = m > 256 ? 64 : (m > 128 ? 32 : 16);
-   const int sub = lane / S, sl = lane - sub * S, CPW = 64 / S;
-   double part = 0.0;
-   for (int j0 = wave * CPW; j0 < K; j0 += NW * CPW) {
-      const int j = j0 + sub;
-      const double* a = A + (long long)(j < K ? j : 0) * lda;
-      double s = 0.0;
-      for (int i0 = 0; i0 < m; i0 += 2 * S * U) {
-         double2 x[U];
+   for (int a0 = wave * CPW; a0 < K; a0 += NW * CPW) {
+      const int j = a0 + sub;
+      double s = 0.0, x[NR];
+      mgs_load(x, A, (unsigned)((j < K ? j : 0) * m + sl), m, S);
+      mgs_mask(x, m, S, sl);
 #pragma unroll
-         for (int u = 0; u < U; u++) {
-            const int i = i0 + 2 * (sl + S * u);
-            x[u] = *(const double2*)(a + (i < m ? i : 0));
-         }
-#pragma unroll
-         for (int u = 0; u < U; u++) {
-            const int i = i0 + 2 * (sl + S * u);
-            const double p = i < m ? x[u].x : 0.0, q = i + 1 < m ? x[u].y : 0.0;
-            s = fma(p, p, s);
-            s = fma(q, q, s);
-         }
-      }
+      for (int t = 0; t < NR; t++) s = fma(x[t], x[t], s);
       s = seg_sum(s, S);
       if (j < K && sl == 0) {
          n2[j] = s;
          order[j] = j;
          act[j] = j;
-         part += s;
       }
    }
-   const double fro = sqrt(block_total(part, red, NW));
-   const double cut = eps * fro, lim = 0.25 * cut * cut;
+   for (int u = 0; u < NB; u++)
+      for (int i = m + tid; i < ldq; i += NT) qs[u * ldq + i] = 0.0;   // past the last row
+   __syncthreads();
+   const double cut = eps * mgs_frobenius(n2, K), lim = 0.25 * cut * cut;
    int k = 0, b = 0, nact = K;
-   double mx0 = 0.0;
-   while (k < kmax) {
-      // the pivot among the positions k..K-1
-      double bv = 0.0;
-      int bp = 0x7fffffff;
-      for (int p = k + tid; p < K; p += MGS_BT) {
-         const double x = n2[order[p]];
+   for (; k < kmax; k++) {
+      double y[NR];
+      int jy = 0;
+      auto load = [&](int a0) {
+         jy = act[min(a0 + sub, nact - 1)];
+         mgs_load(y, A, (unsigned)(jy * m + sl), m, S);
+      };
+      if (PRE && nact) load(wave * CPW);
+      // the pivot among the positions k .. K - 1
+      double bv = 0.0, mx;
+      int bp = 0x7fffffff, best;
+      for (int p = k + tid; p < K; p += NT) {
+         const double x = sqrt(n2[order[p]]);
          if (x > bv || (x == bv && p < bp)) {
             bv = x;
             bp = p;
          }
       }
-      double mx = wave_max(bv);
-      int best = wave_min(bv == mx ? bp : 0x7fffffff);
-      if (lane == 0) {
-         red[wave] = mx;
-         redi[wave] = best;
+      block_pivot(bv, bp, NW, wv, wp, mx, best);
+      if (!(mx > 0.0)) best = k;
+      if (k >= 1 && mx < cut) break;   // uniform over the block
+      const int pj = order[best];
+      for (int i = tid; i < m; i += NT) {
+         double x = A[(unsigned)(pj * m + i)];
+         for (int u = 0; u < b; u++) {
+            const double q = qs[u * ldq + i];
+            const double2 r = R[u * K + pj];
+            x = fma(-q, r.y, fma(-q, r.x, x));
+         }
+         x /= mx;
+         qs[b * ldq + i] = x;
+         Q[(long long)k * m + i] = x;
       }
       __syncthreads();
-      mx = red[0];
-      best = redi[0];
-      for (int w = 1; w < NW; w++)
-         if (red[w] > mx || (red[w] == mx && redi[w] < best)) {
-            mx = red[w];
-            best = redi[w];
-         }
-      if (!(mx > 0.0)) best = k;
-      const bool fresh = b == 0;
-      if (fresh) mx0 = mx;
-      const bool fell = !fresh && mx < 1e-4 * mx0;
-      if (k >= 1 && !fell && sqrt(mx) < cut) break;   // uniform over the block
-      if (fell || b == NB) {
-         // end of the block: its directions out of the active columns, four
-         // columns per wave part, norms afresh
-         for (int a0 = wave * CPW * 4; a0 < nact; a0 += NW * CPW * 4) {
-            int j[4];
-            double s[4] = {0.0, 0.0, 0.0, 0.0};
+      if (tid == 0) {
+         order[best] = order[k];
+         order[k] = pj;
+      }
+      const bool last = b + 1 == NB;
+      if (k + 1 < kmax) {
+         // read anew for each sum: kept, they cost 2 NR registers
+         auto q_row = [&]() {
+            int at = b * ldq + sl;
+            asm volatile("" : "+v"(at));
+            return qs + at;
+         };
+         for (int a0 = wave * CPW; a0 < nact; a0 += NW * CPW) {
+            int rows = m, row = sl;
+            asm volatile("" : "+s"(rows), "+v"(row));   // the row tests stay in the loop: hoisted, they cost registers
+            if (!PRE) load(a0);
+            const int j = jy;
+            double x[NR];
 #pragma unroll
-            for (int c = 0; c < 4; c++) {
-               const int ai = a0 + sub * 4 + c;
-               j[c] = ai < nact ? act[ai] : -1;
+            for (int t = 0; t < NR; t++) x[t] = y[t];
+            mgs_mask(x, rows, S, row);
+            if (PRE && a0 + NW * CPW < nact) load(a0 + NW * CPW);
+            for (int u = 0; u < b; u++) {
+               const double2 r = R[u * K + j];
+               const double* qu = qs + u * ldq + sl;
+#pragma unroll
+               for (int t0 = 0; t0 < NR; t0 += G)
+                  if (t0 * S < rows)
+#pragma unroll
+                     for (int t = t0; t < t0 + G; t++) {
+                        const double p = qu[S * t];
+                        x[t] = fma(-p, r.y, fma(-p, r.x, x[t]));
+                     }
             }
-            for (int i = 2 * sl; i < m; i += 2 * S) {
-               double2 x[4];
+            double r1 = 0.0, r2 = 0.0, s = 0.0;
+            const double* qa = q_row();
 #pragma unroll
-               for (int c = 0; c < 4; c++) x[c] = *(const double2*)(A + (long long)max(j[c], 0) * lda + i);
-               for (int t = 0; t < b; t++) {
-                  // q columns are rows apart: not 16-byte aligned for odd rows
-                  const double* q = Q + (long long)(k - b + t) * m + i;
-                  const double q0 = q[0], q1 = i + 1 < m ? q[1] : 0.0;
+            for (int t0 = 0; t0 < NR; t0 += G)
+               if (t0 * S < rows)
 #pragma unroll
-                  for (int c = 0; c < 4; c++) {
-                     const double r = R[(size_t)t * K + max(j[c], 0)];
-                     x[c].x = fma(-r, q0, x[c].x);
-                     x[c].y = fma(-r, q1, x[c].y);
+                  for (int t = t0; t < t0 + G; t++) r1 = fma(qa[S * t], x[t], r1);
+            r1 = seg_sum(r1, S);
+            const double* qc = q_row();
+#pragma unroll
+            for (int t0 = 0; t0 < NR; t0 += G)
+               if (t0 * S < rows)
+#pragma unroll
+                  for (int t = t0; t < t0 + G; t++) {
+                     const double q = qc[S * t];
+                     x[t] = fma(-q, r1, x[t]);
+                     r2 = fma(q, x[t], r2);
                   }
-               }
+            r2 = seg_sum(r2, S);
+            const double* qd = q_row();
 #pragma unroll
-               for (int c = 0; c < 4; c++) {
-                  if (i + 1 >= m) x[c].y = 0.0;
-                  if (j[c] >= 0) *(double2*)(A + (long long)j[c] * lda + i) = x[c];
-                  s[c] = fma(x[c].x, x[c].x, s[c]);
-                  s[c] = fma(x[c].y, x[c].y, s[c]);
-               }
-            }
+            for (int t0 = 0; t0 < NR; t0 += G)
+               if (t0 * S < rows)
 #pragma unroll
-            for (int c = 0; c < 4; c++) {
-               const double t = seg_sum(s[c], S);
-               if (j[c] >= 0 && sl == 0) n2[j[c]] = t;
+                  for (int t = t0; t < t0 + G; t++) {
+                     x[t] = fma(-qd[S * t], r2, x[t]);
+                     s = fma(x[t], x[t], s);
+                  }
+            s = seg_sum(s, S);
+            if (a0 + sub < nact) {
+               if (sl == 0) {
+                  R[b * K + j] = make_double2(r1, r2);
+                  n2[j] = s;
+               }
+               if (last) {
+#pragma unroll
+                  for (int t = 0; t < NR; t++)
+                     if (row < rows - S * t) (A + S * t)[(unsigned)(j * m + row)] = x[t];
+               }
             }
          }
-         __syncthreads();
-         // positions k.. above the limit stay active
+      }
+      __syncthreads();
+      b++;
+      if (last) {
+         // the columns at positions k + 1 .. that may still be pivots
          if (wave == 0) {
             int cnt = 0;
-            for (int p0 = k; p0 < K; p0 += 64) {
+            for (int p0 = k + 1; p0 < K; p0 += 64) {
                const int p = p0 + lane, j = p < K ? order[p] : 0;
                const bool on = p < K && !(n2[j] < lim);
                const unsigned long long mask = __ballot(on);
@@ -476,105 +636,87 @@ __global__ void __launch_bounds__(MGS_BT) k_mgs_blk(const MgsDesc* __restrict__ 
          __syncthreads();
          nact = s_nact;
          b = 0;
-         continue;
       }
-      const int pj = order[best];
-      const double* ap = A + (long long)pj * lda;
-      // the pivot's residual
-      for (int i = tid; i < m; i += MGS_BT) {
-         double x = ap[i];
-         const double* q = Q + (long long)(k - b) * m + i;
-         const double* r = R + pj;
-#pragma unroll 4
-         for (int t = 0; t < b; t++) {
-            x = fma(-*r, *q, x);
-            q += m;
-            r += K;
+   }
+   if (tid == 0) ranks[d.rank_slot] = k;
+}
+
+// Any other size: the columns read three times and written once a step, their
+// squared norms and order in memory (n2, order: ws_off).
+constexpr int MGS_LT = 1024;
+__host__ __device__ inline size_t mgs_long_bytes(int cols) {
+   return (sizeof(double) + sizeof(int)) * (size_t)(cols + 1) / 16 * 16 + 16;
+}
+__global__ void __launch_bounds__(MGS_LT) k_mgs_long(const MgsDesc* __restrict__ descs, const int* __restrict__ list,
+                                                     double* __restrict__ Abuf, double* __restrict__ Qbuf,
+                                                     int* __restrict__ ranks, double eps,
+                                                     unsigned char* __restrict__ scratch) {
+   __shared__ double wv[MGS_LT / 64];
+   __shared__ int wp[MGS_LT / 64];
+   constexpr int NW = MGS_LT / 64;
+   const MgsDesc d = descs[list[blockIdx.x]];
+   const int m = d.rows, K = d.cols, S = d.seg, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+   const int sub = lane / S, sl = lane - sub * S, CPW = 64 / S, kmax = min(m, K);
+   double* n2 = (double*)(scratch + d.ws_off);
+   int* order = (int*)(n2 + K);
+   for (int a0 = wave * CPW; a0 < K; a0 += NW * CPW) {
+      const int j = a0 + sub;
+      const double* a = Abuf + d.a_off + (long long)(j < K ? j : 0) * m;
+      double s = 0.0;
+      for (int i = sl; i < m; i += S) s = fma(a[i], a[i], s);
+      s = seg_sum(s, S);
+      if (j < K && sl == 0) {
+         n2[j] = s;
+         order[j] = j;
+      }
+   }
+   __syncthreads();
+   const double cut = eps * mgs_frobenius(n2, K), lim = 0.25 * cut * cut;
+   int k = 0;
+   for (; k < kmax; k++) {
+      double bv = 0.0, mx;
+      int bp = 0x7fffffff, best;
+      for (int p = k + tid; p < K; p += MGS_LT) {
+         const double x = sqrt(n2[order[p]]);
+         if (x > bv || (x == bv && p < bp)) {
+            bv = x;
+            bp = p;
          }
-         v[i] = x;
       }
-      if (tid == 0 && mpad > m) v[m] = 0.0;
+      block_pivot(bv, bp, NW, wv, wp, mx, best);
+      if (!(mx > 0.0)) best = k;
+      if (k >= 1 && mx < cut) break;   // uniform over the block
+      const int pj = order[best];
+      double* q = Qbuf + d.q_off + (long long)k * m;
+      for (int i = tid; i < m; i += MGS_LT) q[i] = Abuf[d.a_off + (long long)pj * m + i] / mx;
       __syncthreads();
       if (tid == 0) {
          order[best] = order[k];
          order[k] = pj;
+         n2[pj] = -1.0;   // taken
       }
-      // once more against every earlier direction, eight loads in flight
-      for (int t0 = wave; t0 < k; t0 += NW) {
-         const double* q = Q + (long long)t0 * m;
-         double s0 = 0.0, s1 = 0.0;
-         for (int i0 = 0; i0 < m; i0 += 64 * U) {
-            double x[U];
-#pragma unroll
-            for (int u = 0; u < U; u++) {
-               const int i = i0 + lane + 64 * u;
-               x[u] = q[i < m ? i : 0];
-            }
-#pragma unroll
-            for (int u = 0; u < U; u += 2) {
-               const int i = i0 + lane + 64 * u;
-               s0 = fma(i < m ? x[u] : 0.0, v[i < m ? i : 0], s0);
-               s1 = fma(i + 64 < m ? x[u + 1] : 0.0, v[i + 64 < m ? i + 64 : 0], s1);
-            }
-         }
-         const double s = seg_sum(s0 + s1, 64);
-         if (lane == 0) h[t0] = s;
-      }
-      __syncthreads();
-      double nn = 0.0;
-      for (int i = tid; i < m; i += MGS_BT) {
-         double x = v[i];
-         const double* q = Q + i;
-         int t = 0;
-         for (; t + 7 < k; t += 8, q += 8 * m) {
-            double qv[8];
-#pragma unroll
-            for (int u = 0; u < 8; u++) qv[u] = q[(long long)u * m];
-#pragma unroll
-            for (int u = 0; u < 8; u++) x = fma(-h[t + u], qv[u], x);
-         }
+      for (int a0 = wave * CPW; a0 < K; a0 += NW * CPW) {
+         const int j = a0 + sub;
+         const bool on = j < K && j != pj && !(n2[j] < lim);
+         if (!__any(on)) continue;
+         double* a = Abuf + d.a_off + (long long)(on ? j : pj) * m;
+         double r1 = 0.0, r2 = 0.0, s = 0.0;
 #pragma unroll 4
-         for (; t < k; t++, q += m) x = fma(-h[t], *q, x);
-         v[i] = x;
-         nn = fma(x, x, nn);
-      }
-      const double nrm = sqrt(block_total(nn, red, NW));
-      for (int i = tid; i < m; i += MGS_BT) {
-         const double x = v[i] / nrm;
-         v[i] = x;
-         Q[(long long)k * m + i] = x;
-      }
-      if (tid == 0) n2[pj] = -1.0;
-      __syncthreads();
-      // products of the active columns with q_k
-      for (int a0 = wave * CPW; a0 < nact; a0 += NW * CPW) {
-         const int ai = a0 + sub, j = act[ai < nact ? ai : 0];
-         const double* a = A + (long long)j * lda;
-         double r0 = 0.0, r1 = 0.0;
-         for (int i0 = 0; i0 < m; i0 += 2 * S * U) {
-            double2 x[U];
-#pragma unroll
-            for (int u = 0; u < U; u++) {
-               const int i = i0 + 2 * (sl + S * u);
-               x[u] = *(const double2*)(a + (i < m ? i : 0));
-            }
-#pragma unroll
-            for (int u = 0; u < U; u++) {
-               const int i = i0 + 2 * (sl + S * u);
-               const double2 q = *(const double2*)(v + (i < m ? i : 0));
-               r0 = fma(i < m ? x[u].x : 0.0, q.x, r0);
-               r1 = fma(i + 1 < m ? x[u].y : 0.0, q.y, r1);
-            }
+         for (int i = sl; i < m; i += S) r1 = fma(q[i], a[i], r1);
+         r1 = seg_sum(r1, S);
+#pragma unroll 4
+         for (int i = sl; i < m; i += S) r2 = fma(q[i], fma(-q[i], r1, a[i]), r2);
+         r2 = seg_sum(r2, S);
+#pragma unroll 4
+         for (int i = sl; i < m; i += S) {
+            const double x = fma(-q[i], r2, fma(-q[i], r1, a[i]));
+            if (on) a[i] = x;
+            s = fma(x, x, s);
          }
-         const double r = seg_sum(r0 + r1, S);
-         if (ai < nact && sl == 0) {
-            R[(size_t)b * K + j] = r;
-            if (n2[j] >= 0.0) n2[j] = fma(-r, r, n2[j]);
-         }
+         s = seg_sum(s, S);
+         if (on && sl == 0) n2[j] = s;
       }
       __syncthreads();
-      b++;
-      k++;
    }
    if (tid == 0) ranks[d.rank_slot] = k;
 }
@@ -605,56 +747,82 @@ void launch_gemm_batched(int nbatch, int maxtiles, const GemmDesc* descs, hipStr
       hipLaunchKernelGGL(k_gemm_batched, dim3(maxtiles, nbatch), dim3(256), 0, s, descs);
 }
 
-// The register kernel takes every problem of up to 16 x 64 rows whose column
-// pairs fit its 1024 threads, in launches by the threads they need (small
-// workgroups share a CU); the others go to the blocked kernel, the largest
-// first, its arrays in LDS or, past the LDS, in global scratch.
+// Lanes that share a column's sums (the sums' order: see k_mgs_cols above).
+static int mgs_sum_lanes(int rows, int cols) {
+   if (sizeof(double) * ((size_t)(rows | 1) + 1) * cols <= 96 * 1024) return 1;
+   int S = 4;
+   while (S < 64 && rows > MGS_NR * S) S <<= 1;
+   return S;
+}
+
+// Which kernel takes a problem is settled by rows and cols alone: one lane per
+// column by the rows in registers, two columns a lane group while they fit the
+// threads of a block, else a block that reads the matrix at each step while a
+// column fits a wave's registers.  Small workgroups share a CU, so the launches
+// are by the threads needed.
 void run_mgs(std::vector<MgsDesc>& descs, double* A, double* Q, std::vector<int>& ranks, double eps,
              hipStream_t s) {
-   constexpr size_t LDS_MAX = 158 * 1024;
+   constexpr size_t LDS_MAX = 150 * 1024;   // beside at most 8.2 KB of static LDS
    const int nprob = (int)descs.size();
    ranks.assign(nprob, 0);
    if (nprob == 0) return;
-   constexpr int NC = 5;   // register kernel: 64, 128, 256, 512, 1024 threads
-   std::vector<int> list[NC + 2];
-   size_t lds = 0, ws = 0;
+   struct Class {
+      std::vector<int> list;
+      size_t lds = 0;
+   };
+   // blk: 96, 64, 48, 32 rows a lane, then 16 of 64, 32, 16, 8, 4 lanes; reg:
+   // 1024, 512 threads; cols: by rows in registers, by threads
+   Class large, blk[9], reg[2], cols[3][5];
+   size_t ws = 0;
+   auto put = [](Class& c, int p, size_t lds) {
+      c.list.push_back(p);
+      c.lds = std::max(c.lds, lds);
+   };
    for (int p = 0; p < nprob; p++) {
       MgsDesc& d = descs[p];
-      if ((d.lda & 1) || (d.a_off & 1) || d.lda < d.rows) throw std::runtime_error("sampled matrix not 16-byte aligned");
-      int S = 1;
-      while (S < 64 && d.rows > MGS_NR * S) S <<= 1;
+      const int S = mgs_sum_lanes(d.rows, d.cols);
       d.seg = S;
       const long long threads = (long long)S * ((d.cols + 1) / 2);
-      if (d.rows <= MGS_NR * S && threads <= 1024) {
+      const int n = d.rows <= 32 ? 0 : (d.rows <= 64 ? 1 : 2);
+      const size_t lds = mgs_cols_bytes(d.rows, d.cols, n == 0 ? 32 : (n == 1 ? 64 : 96));
+      if (S == 1 && d.cols <= 1024 && lds <= LDS_MAX) {
          int c = 0;
-         while ((64 << c) < threads) c++;
-         list[c].push_back(p);
+         while ((64 << c) < d.cols) c++;
+         put(cols[n][c], p, lds);
          continue;
       }
-      d.nb = 8;
-      while (d.nb > 2 && mgs_blk_bytes(d.rows, d.cols, d.nb) > LDS_MAX) d.nb >>= 1;
-      const size_t need = mgs_blk_bytes(d.rows, d.cols, d.nb);
-      if (need > LDS_MAX) {
-         d.nb = 8;
-         d.ws_off = (long long)ws;
-         ws += (mgs_blk_bytes(d.rows, d.cols, d.nb) + 15) / 16 * 16;
-         list[NC + 1].push_back(p);
-      } else {
-         lds = std::max(lds, need);
-         list[NC].push_back(p);
+      if (S > 1 && d.rows <= MGS_NR * S && threads <= 1024) {
+         put(reg[threads <= 512 ? 1 : 0], p, 0);
+         continue;
       }
+      constexpr int rows_a_lane[4] = {96, 64, 48, 32};
+      int c = d.rows <= 32 * S ? 3 : (d.rows <= 48 * S ? 2 : (d.rows <= 64 * S ? 1 : 0));
+      if (d.rows <= MGS_NR * S) c = S == 64 ? 4 : (S == 32 ? 5 : (S == 16 ? 6 : (S == 8 ? 7 : 8)));
+      const int nrs = (c < 4 ? rows_a_lane[c] : MGS_NR) * S;
+      d.nb = 4;
+      while (d.nb > 1 && mgs_blk_bytes(nrs, d.cols, d.nb) > LDS_MAX) d.nb >>= 1;
+      // (the kernel's offsets into a matrix are 32 bits)
+      if (S > 1 && d.rows <= nrs && mgs_blk_bytes(nrs, d.cols, d.nb) <= LDS_MAX) {
+         put(blk[c], p, mgs_blk_bytes(nrs, d.cols, d.nb));
+         continue;
+      }
+      d.ws_off = (long long)ws;
+      ws += mgs_long_bytes(d.cols);
+      put(large, p, 0);
    }
-   for (int c = NC; c < NC + 2; c++)
-      std::stable_sort(list[c].begin(), list[c].end(), [&](int x, int y) {
-         return (long long)descs[x].lda * descs[x].cols > (long long)descs[y].lda * descs[y].cols;
+   // the largest ahead: they run longest
+   auto longest_first = [&](Class& c) {
+      std::stable_sort(c.list.begin(), c.list.end(), [&](int x, int y) {
+         return (long long)descs[x].rows * descs[x].cols > (long long)descs[y].rows * descs[y].cols;
       });
-   std::vector<int> all;
-   size_t at[NC + 3];
-   for (int c = 0; c < NC + 2; c++) {
-      at[c] = all.size();
-      all.insert(all.end(), list[c].begin(), list[c].end());
-   }
-   at[NC + 2] = all.size();
+   };
+   longest_first(large);
+   for (Class& c : blk) longest_first(c);
+   std::vector<int> all(large.list);
+   for (const Class& c : blk) all.insert(all.end(), c.list.begin(), c.list.end());
+   for (const Class& c : reg) all.insert(all.end(), c.list.begin(), c.list.end());
+   for (const auto& n : cols)
+      for (const Class& c : n) all.insert(all.end(), c.list.begin(), c.list.end());
    DBuf<MgsDesc> dd;
    DBuf<int> dl, dr;
    DBuf<unsigned char> dws;
@@ -662,40 +830,48 @@ void run_mgs(std::vector<MgsDesc>& descs, double* A, double* Q, std::vector<int>
    dl.upload(all, s);
    dr.alloc(nprob);
    if (ws) dws.alloc(ws);
+   auto k96 = k_mgs_blk<96, 64, 512, false>, k64 = k_mgs_blk<64, 64, 512, false>;
+   auto k48 = k_mgs_blk<48, 64, 768, false>, k32 = k_mgs_blk<32, 64, 1024, false>;
+   decltype(k96) k16[5] = {k_mgs_blk<16, 64, 1024, true>, k_mgs_blk<16, 32, 1024, true>, k_mgs_blk<16, 16, 1024, true>,
+                           k_mgs_blk<16, 8, 1024, true>, k_mgs_blk<16, 4, 1024, true>};
    static std::once_flag attr;
-   std::call_once(attr, [] {
-      FSVD_CHECK(hipFuncSetAttribute((const void*)k_mgs_blk<false>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                     (int)LDS_MAX));
+   std::call_once(attr, [&] {
+      for (const void* k : {(const void*)k96, (const void*)k64, (const void*)k48, (const void*)k32,
+                            (const void*)k16[0], (const void*)k16[1], (const void*)k16[2], (const void*)k16[3],
+                            (const void*)k16[4], (const void*)k_mgs_cols<32>, (const void*)k_mgs_cols<64>,
+                            (const void*)k_mgs_cols<96>})
+         FSVD_CHECK(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)LDS_MAX));
    });
-   // the blocked problems first: they run longest
-   for (int c = NC + 1; c >= 0; c--) {
-      const unsigned n = (unsigned)(at[c + 1] - at[c]);
-      const int* l = dl.p + at[c];
-      if (!n) continue;
-      switch (c) {
-         case 0: hipLaunchKernelGGL(k_mgs_reg<64>, dim3(n), dim3(64), 0, s, dd.p, l, A, Q, dr.p, eps); break;
-         case 1: hipLaunchKernelGGL(k_mgs_reg<128>, dim3(n), dim3(128), 0, s, dd.p, l, A, Q, dr.p, eps); break;
-         case 2: hipLaunchKernelGGL(k_mgs_reg<256>, dim3(n), dim3(256), 0, s, dd.p, l, A, Q, dr.p, eps); break;
-         case 3: hipLaunchKernelGGL(k_mgs_reg<512>, dim3(n), dim3(512), 0, s, dd.p, l, A, Q, dr.p, eps); break;
-         case 4: hipLaunchKernelGGL(k_mgs_reg<1024>, dim3(n), dim3(1024), 0, s, dd.p, l, A, Q, dr.p, eps); break;
-         case 5:
-            hipLaunchKernelGGL(k_mgs_blk<false>, dim3(n), dim3(MGS_BT), lds, s, dd.p, l, A, Q, dr.p, eps, nullptr);
-            break;
-         default:
-            hipLaunchKernelGGL(k_mgs_blk<true>, dim3(n), dim3(MGS_BT), 0, s, dd.p, l, A, Q, dr.p, eps, dws.p);
-            break;
-      }
-   }
+   const int* l = dl.p;
+   if (!large.list.empty())
+      hipLaunchKernelGGL(k_mgs_long, dim3((unsigned)large.list.size()), dim3(MGS_LT), 0, s, dd.p, l, A, Q, dr.p, eps,
+                         dws.p);
+   l += large.list.size();
+   auto launch = [&](auto kernel, const Class& c, int threads) {
+      const unsigned n = (unsigned)c.list.size();
+      if (n) hipLaunchKernelGGL(kernel, dim3(n), dim3(threads), c.lds, s, dd.p, l, A, Q, dr.p, eps);
+      l += n;
+   };
+   launch(k96, blk[0], 512);
+   launch(k64, blk[1], 512);
+   launch(k48, blk[2], 768);
+   launch(k32, blk[3], 1024);
+   for (int c = 0; c < 5; c++) launch(k16[c], blk[4 + c], 1024);
+   launch(k_mgs_reg<1024>, reg[0], 1024);
+   launch(k_mgs_reg<512>, reg[1], 512);
+   for (int c = 0; c < 5; c++) launch(k_mgs_cols<32>, cols[0][c], 64 << c);
+   for (int c = 0; c < 5; c++) launch(k_mgs_cols<64>, cols[1][c], 64 << c);
+   for (int c = 0; c < 5; c++) launch(k_mgs_cols<96>, cols[2][c], 64 << c);
    FSVD_CHECK(hipGetLastError());
    std::vector<int> h(nprob);
    FSVD_CHECK(hipMemcpyAsync(h.data(), dr.p, sizeof(int) * nprob, hipMemcpyDeviceToHost, s));
    FSVD_CHECK(hipStreamSynchronize(s));
    for (int i = 0; i < nprob; i++) ranks[descs[i].rank_slot] = h[descs[i].rank_slot];
    if (const char* e = std::getenv("FFTSVD_TIMING"); e && e[0] == '1') {
-      std::fprintf(stderr, "[fftsvd mgs] %d problems: in registers", nprob);
-      for (int c = 0; c < NC; c++) std::fprintf(stderr, " %zu", list[c].size());
-      std::fprintf(stderr, " (64..1024 threads), blocked %zu + %zu\n", list[NC].size(),
-                   list[NC + 1].size());
+      std::fprintf(stderr, "[fftsvd mgs] %d problems: %zu large, blocked", nprob, large.list.size());
+      for (const Class& c : blk) std::fprintf(stderr, " %zu", c.list.size());
+      std::fprintf(stderr, ", in registers %zu %zu, the others a lane per column\n", reg[0].list.size(),
+                   reg[1].list.size());
    }
 }
 

@@ -1375,17 +1375,16 @@ std::unique_ptr<TreeOp> build_tree_op(const double* pan_cent, int npan, const Pa
                      int idx = t.cube_pt_sorted[off + (unsigned)p * (unsigned)I.nq / (unsigned)P.pass];
                      for (int d = 0; d < 3; d++) bpts.push_back(pts[3 * (size_t)idx + d]);
                   }
-               // column-major A (np x K, columns lda apart): sample s of layer L at column L*half + s
+               // column-major A (np x K): sample s of layer L at column L*half + s
                b.npt = half;
                b.npan = c.np;
                b.pt_off = base;
                b.pan_off = c.p0;
                m.rows = c.np;
                m.cols = K;
-               m.lda = (c.np + 1) / 2 * 2;
-               b.ld_pt = m.lda;
+               b.ld_pt = c.np;
                b.ld_pan = 1;
-               b.layer_stride = layers == 2 ? (long long)half * m.lda : -1;
+               b.layer_stride = layers == 2 ? (long long)half * c.np : -1;
             } else {
                int base = (int)bpan.size();
                for (int p = 0; p < P.pass; p++)
@@ -1401,19 +1400,18 @@ std::unique_ptr<TreeOp> build_tree_op(const double* pan_cent, int npan, const Pa
                b.pan_off = base;
                m.rows = c.nq;
                m.cols = K;
-               m.lda = (c.nq + 1) / 2 * 2;
                b.ld_pt = 1;
-               b.ld_pan = m.lda;
-               b.layer_stride = layers == 2 ? (long long)half * m.lda : -1;
+               b.ld_pan = c.nq;
+               b.layer_stride = layers == 2 ? (long long)half * c.nq : -1;
             }
             push_blocks(blocks, b);
             mgs.push_back(m);
-            asz += (long long)m.lda * m.cols;
+            asz += (long long)m.rows * m.cols;
             qsz += (long long)m.rows * std::min(m.rows, m.cols);
          }
          auto Abuf = std::make_shared<DBuf<double>>();
          auto Qbuf = std::make_shared<DBuf<double>>();
-         Abuf->alloc(std::max<long long>(asz, 1));
+         Abuf->alloc(asz + MGS_SLACK);
          Qbuf->alloc(std::max<long long>(qsz, 1));
          run_integrals(blocks, bpts, bpan, d_panels, kernel, kappa, Abuf->p, s);
          FSVD_CHECK(hipStreamSynchronize(s));
