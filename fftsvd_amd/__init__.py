@@ -50,6 +50,7 @@ _SIGS = {
     "fftsvd_problem_solve_adjoint": (C.c_int, [_vp, C.c_int, _dp, _dp, C.c_double, C.c_int, _ip, _dp]),
     "fftsvd_problem_grad_kappa": (C.c_int, [_vp, C.c_int, _dp, C.c_double, C.c_int, _dp, _ip]),
     "fftsvd_set_autotune": (C.c_int, [C.c_int]),
+    "fftsvd_release_memory": (C.c_int, [C.POINTER(C.c_longlong)]),
     "fftsvd_translation_params": (C.c_int, [_ip, _ip, _ip, _ip, _dp]),
     "fftsvd_problem_grad_charges": (C.c_int, [_vp, C.c_int, _dp, C.c_double, C.c_int, _dp, _ip]),
     "fftsvd_qual_create": (C.c_int, [_dp, C.c_int, _dp, _dp, C.c_int, C.c_double, C.c_double, C.c_int, C.c_int,
@@ -131,6 +132,14 @@ def lds_bandwidth(width=8, nrep=5):
     g = C.c_double()
     _check(lib().fftsvd_lds_bandwidth(int(width), int(nrep), C.byref(g)))
     return g.value
+
+
+def release_memory():
+    """Give device memory that no problem uses any more back to the device
+    (fftsvd_release_memory); returns the bytes."""
+    n = C.c_longlong()
+    _check(lib().fftsvd_release_memory(C.byref(n)))
+    return n.value
 
 
 def set_autotune(on):

@@ -604,6 +604,13 @@ int fftsvd_set_autotune(int on) {
    API_CATCH
 }
 
+int fftsvd_release_memory(long long* bytes) {
+   API_TRY
+   const size_t n = dev_trim();
+   if (bytes) *bytes = (long long)n;
+   API_CATCH
+}
+
 int fftsvd_translation_params(int* mode, int* budget, int* tile, int* tuned, double* tuned_ms) {
    API_TRY
    bool t = false;

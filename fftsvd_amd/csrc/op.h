@@ -14,10 +14,12 @@ namespace fsvd {
 
 // Device memory for the buffers below (devmem.cpp): blocks given back are
 // kept (bounded) and taken again, so a block must be idle when it is given
-// back; dev_built tells that a problem has been built.
+// back; dev_built tells that a problem has been built; dev_trim gives all that
+// is kept back to the device.
 void* dev_take(size_t bytes);
 void dev_give(void* p);
 void dev_built();
+size_t dev_trim();
 
 // A device buffer that frees itself.  No work that uses it may be in flight
 // when it is destroyed or allocated anew.

@@ -248,6 +248,13 @@ void fftsvd_free(void* p);
  * time per launch.  No counterpart in the reference. */
 int fftsvd_set_autotune(int on);
 int fftsvd_translation_params(int* mode, int* budget, int* tile, int* tuned, double* tuned_ms);
+/* Device memory that destroyed problems and temporaries no longer use is kept
+ * for later calls, at most 1/24 of a device's memory (12 GB of 288); problems
+ * built later take it, and give back what the last two builds left unused.
+ * fftsvd_release_memory gives all of it back now, for other users of the
+ * device (*bytes, if not NULL: how much).  Memory of problems that still exist
+ * stays with them.  Safe from any thread. */
+int fftsvd_release_memory(long long* bytes);
 /* Precision used by solveSurfaceOperator (0 FP64, 1 mixed); default 0. */
 int fftsvd_set_precision(int precision);
 

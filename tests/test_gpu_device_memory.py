@@ -1,7 +1,7 @@
 """Kept device memory (devmem.cpp): problems built, used and destroyed in turn
 and on several threads at once, in blocks that earlier ones gave back, give the
-same bits; memory kept from a large problem goes back to the device once later
-builds have not taken it."""
+same bits; memory kept from a large problem goes back to the device once later builds have
+not taken it, or when it is asked for."""
 import ctypes as C
 import threading
 
@@ -48,22 +48,36 @@ def test_reused_blocks_same_results(threads):
     assert not bad
 
 
-def test_kept_memory_goes_back():
+def _memory():
     fa.lib()
     hip = C.CDLL("libamdhip64.so.7")
     hip.hipMemGetInfo.argtypes = [C.POINTER(C.c_size_t), C.POINTER(C.c_size_t)]
+    f, t = C.c_size_t(), C.c_size_t()
+    assert hip.hipMemGetInfo(C.byref(f), C.byref(t)) == 0
+    return f.value, t.value
 
-    def free():
-        f, t = C.c_size_t(), C.c_size_t()
-        assert hip.hipMemGetInfo(C.byref(f), C.byref(t)) == 0
-        return f.value, t.value
 
+def _free():
+    return _memory()[0]
+
+
+def test_kept_memory_goes_back():
     for _ in range(4):
         _pass(2, 0.124)
-    base, total = free()
+    base, total = _memory()
     _pass(5, 0.124)   # 20480 panels: more than 1 GB
-    kept = base - free()[0]
-    assert kept <= total // 24 + (64 << 20)
+    kept = base - _free()
+    assert 512 << 20 < kept <= total // 24 + (64 << 20)
     for _ in range(4):
         _pass(2, 0.124)
-    assert base - free()[0] <= 256 << 20
+    assert base - _free() <= 256 << 20
+
+
+def test_release_memory():
+    _pass(4, 0.124)
+    before = _free()
+    n = fa.release_memory()
+    assert n > 128 << 20
+    # blocks are whole pages for the runtime
+    assert _free() - before >= n // 2
+    assert fa.release_memory() == 0
