@@ -1,8 +1,10 @@
 """Kept device memory (devmem.cpp): problems built, used and destroyed in turn
 and on several threads at once, in blocks that earlier ones gave back, give the
-same bits; memory kept from a large problem goes back to the device once later builds have
+same bits, also where every block is filled with NaN before it is handed out;
+memory kept from a large problem goes back to the device once later builds have
 not taken it, or when it is asked for."""
 import ctypes as C
+import os
 import threading
 
 import numpy as np
@@ -46,6 +48,24 @@ def test_reused_blocks_same_results(threads):
     for t in th:
         t.join()
     assert not bad
+
+
+@pytest.mark.parametrize("threads", [1, 3])
+def test_filled_blocks_same_results(threads):
+    cases = [(2, 0.124), (3, 0.0), (4, 0.2)]
+    first = [_pass(*c) for c in cases]
+    got = {}
+    os.environ["FFTSVD_FILL_MEMORY"] = "1"
+    try:
+        th = [threading.Thread(target=lambda t=t: got.update({t: [_pass(*c) for c in cases]})) for t in range(threads)]
+        for t in th:
+            t.start()
+        for t in th:
+            t.join()
+    finally:
+        del os.environ["FFTSVD_FILL_MEMORY"]
+    for t in range(threads):
+        assert all(_same(a, b) for a, b in zip(got[t], first))
 
 
 def _memory():
