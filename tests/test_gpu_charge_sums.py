@@ -1,13 +1,19 @@
-"""Charge right-hand sides, reaction potentials and their transposes against
-plain sums over charges and panels, at charge counts around a wave's 64 lanes,
-panel counts around a block's 256 and column counts around one pass (8, 16, 32,
-64).  FP64 sums in another order: 1e-13 of the sum of absolute values; the
-panel integrals are the library's own, one pair at a time.  A charge on a
-centroid with value zero adds nothing to the right-hand side."""
+"""Charge right-hand sides and reaction potentials against plain sums over
+charges and panels, at charge counts around a wave's 64 lanes, panel counts
+around a block's 256 and column counts around one pass (8, 16, 32, 64).  FP64
+sums in another order: 1e-13 of the sum of absolute values; the panel integrals
+are the library's own, one pair at a time.  A charge on a centroid with value
+zero adds nothing to the right-hand side.
+
+Their transposes (collection and right-hand side) through the charge gradient
+1/2 (C x + B^T lambda), A^T lambda = C^T q, with plain sums for C and B, at charge
+counts around one part of the walk over charges (16) and a wave's lanes.  The
+adjoint solve to 1e-12 of its right-hand side lies between: 1e-9."""
 import numpy as np
 import pytest
 
 import fftsvd_amd as fa
+import oracle
 from fftsvd_amd import meshes
 
 pytestmark = pytest.mark.gpu
@@ -57,6 +63,32 @@ def test_zero_charge_on_a_centroid():
     R = g.rhs_batch(np.stack([q, -q], axis=1))
     for r in (g.rhs(), R[:, 0], -R[:, 1]):
         assert np.linalg.norm(r - h.rhs()) <= 1e-13 * np.linalg.norm(r)
+
+
+@pytest.mark.parametrize("nq", [1, 16, 17, 63, 64, 65, 300])
+@pytest.mark.parametrize("centroid", [False, True])
+def test_transposes(nq, centroid):
+    P, x, rng = _problem(2, nq)
+    n = len(P)
+    cent = P.reshape(n, 3, 3).mean(axis=1)
+    if centroid:   # the charge's own gradient is infinite, the others see its 4 pi term
+        x[nq // 2] = oracle.panel_geom(P[11])["centroid"]
+    q = rng.uniform(-1, 1, nq)
+    g = fa.Problem(P, x, q, 4.0, 80.0, 0.124)
+    sl, dl = fa.integrate(P, x)
+    if centroid:
+        dl[nq // 2, 11] += 4.0 * np.pi
+    C = np.hstack([-dl, sl])
+    sol = rng.uniform(-1, 1, g.nvec)
+    lam, _ = g.solve_adjoint(C.T @ q, 1e-12)
+    grad = g.grad_charges(sol, 1e-12, conversion=g.eps_in)
+    for j in range(nq):
+        if centroid and j == nq // 2:
+            continue
+        w = 1.0 / np.linalg.norm(x[j] - cent, axis=1)
+        ref, mag = 0.5 * (C[j] @ sol + w @ lam[:n]), np.abs(C[j]) @ np.abs(sol) + w @ np.abs(lam[:n])
+        assert abs(grad[j] - ref) <= 1e-9 * mag
+    g.close()
 
 
 @pytest.mark.parametrize("sub,nq", [(1, 5), (3, 65)])
