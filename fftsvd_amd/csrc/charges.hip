@@ -11,10 +11,13 @@
 //   - sums over charges (right-hand sides, transposed potentials): a wave has
 //     64 panels on its lanes, the part of their records that the moment
 //     expansion needs in registers, and walks through charges (scalar loads).
-// The walked range is split over blocks until the chip is full, whatever nq,
-// ne and ncol are; the parts' sums go to ws and a second launch adds them in
-// order.  The split depends on nq and ne alone, so a column's result does not
-// depend on the other columns.  Kernel times before and after (one block per
+// The walked range is split over blocks until the chip is full; the parts' sums
+// go to ws and a second launch adds them in order.  The split depends on nq and
+// ne alone, so a column's result does not depend on the other columns.  Not
+// split are the right-hand sides of the surface operator: each panel's charges
+// are one chain, whose rounding a plain sum shares (4e-16 from it; in parts
+// 8e-16, 30 000 panels and 500 charges), so a small surface fills few blocks
+// (1280 panels: 5).  Kernel times before and after (one block per
 // charge or 256 panels, the record read from memory for each pair, a division
 // per column): potentials of 2000 charges and 100 000 panels 9.5 to 2.1 ms, of
 // 500 and 30 000 with 64 columns 5.5 to 1.8 ms; right-hand sides for the latter
@@ -127,7 +130,7 @@ __global__ void __launch_bounds__(256) k_add_parts(long long n, int ns, const do
 
 // --- sums over charges: panels on lanes -------------------------------------
 // part[(sp * ncol + col) * ne + e], block (256 panels, part sp); with one part
-// (ns = 1) the result itself.
+// (ns = 1, always for SUM_RHS) the result itself.
 
 enum { SUM_RHS, SUM_QUAL, SUM_COLLECT };
 
@@ -217,7 +220,7 @@ __global__ void __launch_bounds__(256) k_panel_sums(int ne, int nq, int ncol, in
 #pragma unroll
    for (int c = 0; c < NS; c++) {
       if (col0 + c >= nc) break;
-      if (ns == 1)
+      if (MODE == SUM_RHS || ns == 1)
          panel_result<MODE>(e, col0 + c, s[c], idx, fourpe, ldr, y, y2);
       else
          part[((size_t)sp * nc + col0 + c) * ne + e] = s[c];
@@ -258,14 +261,12 @@ double* room(DBuf<double>& ws, size_t n) {
 template <int MODE>
 void panel_sums(int ne, int nq, int ncol, const double* cent, const PanelGeom* panels, const int* idx,
                 const int* self_ok, const double* qpos, const double* q, double fourpe, long long ldr, double* y,
-                double* y2, DBuf<double>& ws, hipStream_t s) {
+                double* y2, DBuf<double>* ws, hipStream_t s) {
    if (ne <= 0 || ncol <= 0) return;
-   // right-hand sides: the charges in one chain, whose rounding a plain sum
-   // shares (4e-16 from it; in parts 8e-16, 30 000 panels and 500 charges)
    const Split w = split_walk((ne + 255) / 256, nq, MODE == SUM_RHS ? std::max(nq, 1) : 16);
    for (int c0 = 0; c0 < ncol; c0 += COL_CHUNK) {
       const int nc = std::min(COL_CHUNK, ncol - c0), np = MODE == SUM_COLLECT ? 2 : nc;
-      double* part = w.parts > 1 ? room(ws, (size_t)w.parts * np * ne) : nullptr;
+      double* part = MODE != SUM_RHS && w.parts > 1 ? room(*ws, (size_t)w.parts * np * ne) : nullptr;
       const double* qc = q + (size_t)c0 * nq;
       double* yc = y + (size_t)c0 * ldr;
       constexpr int NB = MODE == SUM_COLLECT ? 1 : 16;
@@ -276,24 +277,25 @@ void panel_sums(int ne, int nq, int ncol, const double* cent, const PanelGeom* p
          hipLaunchKernelGGL((k_panel_sums<MODE, NB>), dim3(w.groups * w.parts, (nc + NB - 1) / NB), dim3(256), 0, s,
                             ne, nq, nc, w.groups, w.parts, w.per, cent, panels, idx, self_ok, qpos, qc, fourpe, ldr,
                             part, yc, y2);
-      if (w.parts > 1)
-         hipLaunchKernelGGL((k_panel_parts<MODE>), dim3((ne + 255) / 256, np), dim3(256), 0, s, ne, np, w.parts, part,
-                            idx, fourpe, ldr, yc, y2);
+      if constexpr (MODE != SUM_RHS)
+         if (w.parts > 1)
+            hipLaunchKernelGGL((k_panel_parts<MODE>), dim3((ne + 255) / 256, np), dim3(256), 0, s, ne, np, w.parts,
+                               part, idx, fourpe, ldr, yc, y2);
    }
 }
 }  // namespace
 
 void launch_rhs(int ne, const double* cent, const int* out, int nq, int ncol, const double* qpos, const double* q,
-                long long ldr, double* rhs, DBuf<double>& ws, hipStream_t s) {
-   panel_sums<SUM_RHS>(ne, nq, ncol, cent, nullptr, out, nullptr, qpos, q, 0.0, ldr, rhs, nullptr, ws, s);
+                long long ldr, double* rhs, hipStream_t s) {
+   panel_sums<SUM_RHS>(ne, nq, ncol, cent, nullptr, out, nullptr, qpos, q, 0.0, ldr, rhs, nullptr, nullptr, s);
 }
 void launch_qual_rhs(int n, const PanelGeom* panels, int nq, int ncol, const double* qpos, const double* q,
                      double fourpe, long long ldr, double* rhs, DBuf<double>& ws, hipStream_t s) {
-   panel_sums<SUM_QUAL>(n, nq, ncol, nullptr, panels, nullptr, nullptr, qpos, q, fourpe, ldr, rhs, nullptr, ws, s);
+   panel_sums<SUM_QUAL>(n, nq, ncol, nullptr, panels, nullptr, nullptr, qpos, q, fourpe, ldr, rhs, nullptr, &ws, s);
 }
 void launch_collect_t(int ne, const PanelGeom* panels, const int* pidx, const int* self_ok, int nq, const double* qpos,
                       const double* q, double* ssl, double* sdl, DBuf<double>& ws, hipStream_t s) {
-   panel_sums<SUM_COLLECT>(ne, nq, 1, nullptr, panels, pidx, self_ok, qpos, q, 0.0, 0, ssl, sdl, ws, s);
+   panel_sums<SUM_COLLECT>(ne, nq, 1, nullptr, panels, pidx, self_ok, qpos, q, 0.0, 0, ssl, sdl, &ws, s);
 }
 
 void launch_potentials(int nq, int ne, int ncol, const PanelGeom* panels, const int* pidx, const double* coef,

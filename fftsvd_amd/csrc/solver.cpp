@@ -67,7 +67,7 @@ void launch_precond_t(int nb, const int* ia, const int* ib, const double* M, con
 // sums over charges and panels, ncol columns at once; ws: room for partial
 // sums, which has to live until s has drained
 void launch_rhs(int ne, const double* cent, const int* out, int nq, int ncol, const double* qpos, const double* q,
-                long long ldr, double* rhs, DBuf<double>& ws, hipStream_t s);
+                long long ldr, double* rhs, hipStream_t s);
 void launch_qual_rhs(int n, const PanelGeom* panels, int nq, int ncol, const double* qpos, const double* q,
                      double fourpe, long long ldr, double* rhs, DBuf<double>& ws, hipStream_t s);
 void launch_potentials(int nq, int ne, int ncol, const PanelGeom* panels, const int* pidx, const double* coef,
@@ -803,11 +803,11 @@ void problem_rhs(Problem& pr, double* rhs) {
             out.push_back(C.startdphi + j);
          }
       }
-      DBuf<double> dc, ws;
+      DBuf<double> dc;
       DBuf<int> dout;
       dc.upload(cent, s);
       dout.upload(out, s);
-      launch_rhs((int)out.size(), dc.p, dout.p, (int)pr.q.size(), 1, pr.d_qpos.p, pr.d_q.p, pr.nvec, rhs, ws, s);
+      launch_rhs((int)out.size(), dc.p, dout.p, (int)pr.q.size(), 1, pr.d_qpos.p, pr.d_q.p, pr.nvec, rhs, s);
       FSVD_CHECK(hipStreamSynchronize(s));
    }
 }
@@ -841,11 +841,11 @@ void problem_rhs_batch(Problem& pr, int ncol, const double* q, double* rhs) {
             out.push_back(C.startdphi + j);
          }
       }
-      DBuf<double> dc, ws;
+      DBuf<double> dc;
       DBuf<int> dout;
       dc.upload(cent, s);
       dout.upload(out, s);
-      launch_rhs((int)out.size(), dc.p, dout.p, nq, ncol, pr.d_qpos.p, q, pr.nvec, rhs, ws, s);
+      launch_rhs((int)out.size(), dc.p, dout.p, nq, ncol, pr.d_qpos.p, q, pr.nvec, rhs, s);
       FSVD_CHECK(hipStreamSynchronize(s));
    }
 }
