@@ -1794,10 +1794,6 @@ static void build_trans_plan(TreeOp& op, hipStream_t s) {
    // target cubes project their points, point-major U in the place of VT
    std::vector<ProjChunk> chunks;
    std::vector<SrcPlan> src;
-   std::vector<TransDesc> tr;
-   long long ut_n = 0;
-   for (const FarLevel& lv : op.levels) ut_n += (long long)lv.UT64.n;
-   P.VTc64.alloc(std::max<long long>(ut_n, 1));
    // source cubes receive: both layers' rows of PV in the place of UTI
    std::vector<TgtPlan> tgt;
    std::vector<std::vector<int>> lv_w(L);
@@ -1835,7 +1831,7 @@ static void build_trans_plan(TreeOp& op, hipStream_t s) {
          sp.spec_off = spec_b + (long long)td.spec_slot * pst;
          src.push_back(sp);
          P.maxr_src = std::max(P.maxr_src, td.r);
-         tr.push_back({lv.UT64.p + td.u_off, P.VTc64.p + ut_b + td.u_off, td.r, td.nq});
+         tp->u_blocks.push_back({ut_b + td.u_off, td.r, td.nq});
       }
       tp->lv.push_back({(int)tgt.size(), (int)lv.h_src.size(), lv.pad, pst, lv.ntgt, t_b / 2, spec_b});
       lv_vt[li] = vt_b;
@@ -1870,13 +1866,6 @@ static void build_trans_plan(TreeOp& op, hipStream_t s) {
       t_b += 2LL * 343 * pst;
       spec_b += (long long)lv.ntgt * pst;
       acc_b += (long long)lv.nsrc * pst;
-   }
-   {
-      DBuf<TransDesc> dtr;
-      dtr.upload(tr, s);
-      launch_transpose_batched<double>((int)tr.size(), dtr.p, s);
-      if (op.have32) to_f32(P.VTc64, P.VTc32, s);
-      FSVD_CHECK(hipStreamSynchronize(s));
    }
    P.nchunk = (int)chunks.size();
    P.nsrc = (int)src.size();
@@ -1988,6 +1977,18 @@ static void build_trans_plan(TreeOp& op, hipStream_t s) {
    op.trans = std::move(tp);
 }
 
+// Point-major U of one precision.
+template <typename T>
+static void transpose_u(const TransPlan& tp, const DBuf<T>& U, DBuf<T>& out, hipStream_t s) {
+   out.alloc(std::max<size_t>(U.n, 1));
+   std::vector<TransDesc> tr;
+   for (const UBlock& b : tp.u_blocks) tr.push_back({U.p + b.off, out.p + b.off, b.r, b.nq});
+   DBuf<TransDesc> dtr;
+   dtr.upload(tr, s);
+   launch_transpose_batched<T>((int)tr.size(), dtr.p, s);
+   FSVD_CHECK(hipStreamSynchronize(s));
+}
+
 bool tree_transpose_ready(const TreeOp& op, int prec) {
    return op.trans && (prec == PREC_F32 ? op.trans->have32 : op.trans->have64);
 }
@@ -2000,10 +2001,12 @@ void tree_prepare_transpose(TreeOp& op, int prec, hipStream_t s) {
    TransPlan& tp = *op.trans;
    if (prec == PREC_F32) {
       if (!op.have32) throw std::runtime_error("operator has no FP32 copy");
+      transpose_u(tp, op.plan.UT32, tp.P.VTc32, s);
       build_translate_pipe(tp.P, tp.lv, tp.h_tgt, tp.isrc, tp.itoff, op.stats.pipe);
       make_pipe(tp.P.pipe, tp.P, op.plan.Tsp32.p, s, op.stats.pipe.mode);
       tp.have32 = true;
    } else {
+      transpose_u(tp, op.plan.UT64, tp.P.VTc64, s);
       build_translate_f64(tp.P, tp.lv, tp.h_tgt, tp.isrc, tp.itoff, s);
       tp.have64 = true;
    }

@@ -170,8 +170,13 @@ struct ApplyPlan {
 // with the two sides swapped (point-major U for the projection, UTI in the
 // place of PV and PV in that of UTI, the interaction lists reversed), and the
 // output leaves.  The matrices other than U are the forward plan's.
+struct UBlock {
+   long long off;   // of a target cube's U in the plan's UT, r x nq
+   int r, nq;
+};
 struct TransPlan {
-   ApplyPlan P;   // chunks, src, translation, work vectors, VTc = point-major U
+   ApplyPlan P;   // chunks, src, translation, work vectors, VTc = point-major U of the precisions in use
+   std::vector<UBlock> u_blocks;
    DBuf<TgtPlan> tgt[3];   // the source cubes with the rows of the single layer, the double layer, both
    int ntgt = 0;
    // the translation's lists, for the plans made at the first use of each precision
