@@ -172,8 +172,7 @@ static_assert(TP_TROWS % 4 == 0, "source rows start on an LDS bank-quarter bound
 // T + c * pst), its tree's forward spectra (source k of the tile at
 // spec + gsrc[src_off + k]) and accumulated spectra (octet target
 // outputs at acc + oacc[...]), the union size nsrc, the level's pad and
-// stride.  Tiles carry their pointers, so one launch can cover the
-// translations of several trees.
+// stride.
 struct TpTile {
    const float2* T;
    const float2* spec;

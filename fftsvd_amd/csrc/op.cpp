@@ -1468,7 +1468,6 @@ std::unique_ptr<TreeOp> build_tree_op(const double* pan_cent, int npan, const Pa
             pvs += 2LL * c.rowrank * gp3;
             src_slot[cl[ci]] = sd.spec_slot;
             lv.h_src.push_back(sd);
-            lv.maxr_src = std::max(lv.maxr_src, c.rowrank);
          }
          if (c.nq > 0 && c.colrank > 0) {
             TgtDesc td;
@@ -1482,16 +1481,12 @@ std::unique_ptr<TreeOp> build_tree_op(const double* pan_cent, int npan, const Pa
             utis += (long long)c.colrank * gp3;
             tgt_slot[cl[ci]] = td.spec_slot;
             lv.h_tgt.push_back(td);
-            lv.maxr_tgt = std::max(lv.maxr_tgt, c.colrank);
          }
       }
       lv.VT64.alloc(std::max<long long>(vts, 1));
       lv.PV64.alloc(std::max<long long>(pvs, 1));
       lv.UT64.alloc(std::max<long long>(uts, 1));
       lv.UTI64.alloc(std::max<long long>(utis, 1));
-      for (auto& sd : lv.h_src) {
-         (void)sd;
-      }
       {
          size_t si = 0, ti = 0;
          for (size_t ci = 0; ci < cl.size(); ci++) {
@@ -1559,7 +1554,7 @@ std::unique_ptr<TreeOp> build_tree_op(const double* pan_cent, int npan, const Pa
    }
    tp = now_ms();
    double tm = tp;
-   // interaction lists (Cube_multiply_T, Cube.c:2062-2111) and their transposes
+   // interaction lists (Cube_multiply_T, Cube.c:2062-2111)
    for (FarLevel& lv : op.levels) {
       for (TgtDesc& td : lv.h_tgt) td.nint = 0;
       size_t ti = 0;

@@ -64,7 +64,7 @@ struct DBuf {
 
 struct FarLevel {
    int level = 0, n = 0, pad = 0, gp3 = 0;
-   int nsrc = 0, ntgt = 0, maxr_src = 0, maxr_tgt = 0;
+   int nsrc = 0, ntgt = 0;
    std::vector<SrcDesc> h_src;
    std::vector<TgtDesc> h_tgt;
    std::vector<int> h_isrc, h_itoff;     // target-side interaction lists
@@ -113,7 +113,7 @@ struct PipeHost {
    std::vector<double> cost;
 };
 // The device form: nblk persistent blocks, block b takes the tasks
-// range[b]; one launch of k_translate_pipe.  It may cover several trees.
+// range[b]; one launch of k_translate_pipe over all levels of a tree.
 struct PipeDev {
    int nblk = 0, mode = 1;   // mode: 0 staging through registers, 1 direct global->LDS transfers
    DBuf<int2> range;
