@@ -48,7 +48,7 @@ struct MgsDesc {
    long long q_off;
    int rank_slot;
    int seg;             // lanes that share a column's sums
-   int nb;              // blocked kernel: steps per block
+   int shape, nb;       // blocked kernel: rows a lane x lanes per column, steps per block
    long long ws_off;    // k_mgs_long: its arrays in the scratch
 };
 

@@ -129,15 +129,15 @@ __global__ void __launch_bounds__(256) k_gemm_batched(const GemmDesc* __restrict
 // rounding errors' size.
 //
 // One workgroup runs a problem from its first to its last step, so a batch is
-// a dozen launches at most:
+// a few launches:
 //   k_mgs_cols  one lane per column, columns in registers and LDS
 //   k_mgs_reg   S lanes per two columns, all in registers
 //   k_mgs_blk   larger ones, read from L2 once per step
 //   k_mgs_long  the rest (more than 6144 rows)
 // Against two launches per step over all problems, each reading and writing
-// every matrix: one operator pair's bases take 130 ms of kernel time instead of
-// 212 at 100 000 panels (130 launches instead of 2180), 63 instead of 59 at
-// 31 000; the operators are there after 140 and 64 ms instead of 206 and 105,
+// every matrix: one operator pair's bases take 111 ms of kernel time instead of
+// 212 at 100 000 panels (55 launches instead of 2180), 39 instead of 59 at
+// 31 000; the operators are there after 125 and 57 ms instead of 206 and 105,
 // with the kept device memory.
 
 // Value of another lane of the row by DPP (quad permutations, half-row mirror,
@@ -467,15 +467,10 @@ __host__ __device__ inline size_t mgs_blk_bytes(int NRS, int cols, int nb) {
           (sizeof(double) + 2 * sizeof(int)) * (size_t)cols;
 }
 template <int NR, int S, int NT, bool PRE>
-__global__ void __launch_bounds__(NT) k_mgs_blk(const MgsDesc* __restrict__ descs, const int* __restrict__ list,
-                                                double* __restrict__ Abuf, double* __restrict__ Qbuf,
-                                                int* __restrict__ ranks, double eps) {
-   extern __shared__ __align__(16) unsigned char sm[];
-   __shared__ double wv[NT / 64];
-   __shared__ int wp[NT / 64];
-   __shared__ int s_nact;
+__device__ __forceinline__ void mgs_blk(const MgsDesc& d, double* __restrict__ Abuf, double* __restrict__ Qbuf,
+                                        int* __restrict__ ranks, double eps, unsigned char* sm, double* wv,
+                                        int* wp, int& s_nact) {
    constexpr int NW = NT / 64, G = NR > 32 ? 16 : 4;   // G: reads of q in flight, for few waves more
-   const MgsDesc d = descs[list[blockIdx.x]];
    constexpr int ldq = NR * S;
    const int m = d.rows, K = d.cols, NB = d.nb;
    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -555,7 +550,7 @@ __global__ void __launch_bounds__(NT) k_mgs_blk(const MgsDesc* __restrict__ desc
             return qs + at;
          };
          for (int a0 = wave * CPW; a0 < nact; a0 += NW * CPW) {
-            int rows = m, row = sl;
+            int rows = __builtin_amdgcn_readfirstlane(m), row = sl;
             asm volatile("" : "+s"(rows), "+v"(row));   // the row tests stay in the loop: hoisted, they cost registers
             if (!PRE) load(a0);
             const int j = jy;
@@ -639,6 +634,39 @@ __global__ void __launch_bounds__(NT) k_mgs_blk(const MgsDesc* __restrict__ desc
       }
    }
    if (tid == 0) ranks[d.rank_slot] = k;
+}
+
+// The rows a lane takes and the lanes per column are settled per problem; the
+// problems of all of them share a launch (launches of a stream run one after
+// the other, and a level's are short of problems: a launch per shape made the
+// 31 000-panel operators 64 ms instead of 57): 12 waves with up to 48 rows a
+// lane, 8 waves above, by the registers.
+enum { MGS_16x4, MGS_16x8, MGS_16x16, MGS_16x32, MGS_16x64, MGS_32x64, MGS_48x64, MGS_64x64, MGS_96x64 };
+template <int NT>
+__global__ void __launch_bounds__(NT) k_mgs_blk(const MgsDesc* __restrict__ descs, const int* __restrict__ list,
+                                                double* __restrict__ Abuf, double* __restrict__ Qbuf,
+                                                int* __restrict__ ranks, double eps) {
+   extern __shared__ __align__(16) unsigned char sm[];
+   __shared__ double wv[NT / 64];
+   __shared__ int wp[NT / 64];
+   __shared__ int s_nact;
+   const MgsDesc d = descs[list[blockIdx.x]];
+   if constexpr (NT == 512) {
+      if (d.shape == MGS_64x64)
+         mgs_blk<64, 64, NT, false>(d, Abuf, Qbuf, ranks, eps, sm, wv, wp, s_nact);
+      else
+         mgs_blk<96, 64, NT, false>(d, Abuf, Qbuf, ranks, eps, sm, wv, wp, s_nact);
+   } else {
+      switch (d.shape) {
+         case MGS_16x4: mgs_blk<16, 4, NT, true>(d, Abuf, Qbuf, ranks, eps, sm, wv, wp, s_nact); break;
+         case MGS_16x8: mgs_blk<16, 8, NT, true>(d, Abuf, Qbuf, ranks, eps, sm, wv, wp, s_nact); break;
+         case MGS_16x16: mgs_blk<16, 16, NT, true>(d, Abuf, Qbuf, ranks, eps, sm, wv, wp, s_nact); break;
+         case MGS_16x32: mgs_blk<16, 32, NT, true>(d, Abuf, Qbuf, ranks, eps, sm, wv, wp, s_nact); break;
+         case MGS_16x64: mgs_blk<16, 64, NT, true>(d, Abuf, Qbuf, ranks, eps, sm, wv, wp, s_nact); break;
+         case MGS_32x64: mgs_blk<32, 64, NT, false>(d, Abuf, Qbuf, ranks, eps, sm, wv, wp, s_nact); break;
+         default: mgs_blk<48, 64, NT, false>(d, Abuf, Qbuf, ranks, eps, sm, wv, wp, s_nact); break;
+      }
+   }
 }
 
 // Any other size: the columns read three times and written once a step, their
@@ -758,8 +786,7 @@ static int mgs_sum_lanes(int rows, int cols) {
 // Which kernel takes a problem is settled by rows and cols alone: one lane per
 // column by the rows in registers, two columns a lane group while they fit the
 // threads of a block, else a block that reads the matrix at each step while a
-// column fits a wave's registers.  Small workgroups share a CU, so the launches
-// are by the threads needed.
+// column fits a wave's registers.
 void run_mgs(std::vector<MgsDesc>& descs, double* A, double* Q, std::vector<int>& ranks, double eps,
              hipStream_t s) {
    constexpr size_t LDS_MAX = 150 * 1024;   // beside at most 8.2 KB of static LDS
@@ -770,46 +797,75 @@ void run_mgs(std::vector<MgsDesc>& descs, double* A, double* Q, std::vector<int>
       std::vector<int> list;
       size_t lds = 0;
    };
-   // blk: 96, 64, 48, 32 rows a lane, then 16 of 64, 32, 16, 8, 4 lanes; reg:
-   // 1024, 512 threads; cols: by rows in registers, by threads
-   Class large, blk[9], reg[2], cols[3][5];
+   // blk: 8, 12 waves; reg: 1024, 512 threads; cols: by rows in registers, by threads
+   Class large, blk[2], reg[2], cols[3][5];
+   constexpr int cols_rows[3] = {32, 64, 96};
    size_t ws = 0;
    auto put = [](Class& c, int p, size_t lds) {
       c.list.push_back(p);
       c.lds = std::max(c.lds, lds);
    };
+   auto cols_lds = [&](int p, int n) { return mgs_cols_bytes(descs[p].rows, descs[p].cols, cols_rows[n]); };
    for (int p = 0; p < nprob; p++) {
       MgsDesc& d = descs[p];
       const int S = mgs_sum_lanes(d.rows, d.cols);
       d.seg = S;
-      const long long threads = (long long)S * ((d.cols + 1) / 2);
       const int n = d.rows <= 32 ? 0 : (d.rows <= 64 ? 1 : 2);
-      const size_t lds = mgs_cols_bytes(d.rows, d.cols, n == 0 ? 32 : (n == 1 ? 64 : 96));
-      if (S == 1 && d.cols <= 1024 && lds <= LDS_MAX) {
+      if (S == 1 && d.cols <= 1024 && cols_lds(p, n) <= LDS_MAX) {
          int c = 0;
          while ((64 << c) < d.cols) c++;
-         put(cols[n][c], p, lds);
+         put(cols[n][c], p, cols_lds(p, n));
          continue;
       }
+      const long long threads = (long long)S * ((d.cols + 1) / 2);
       if (S > 1 && d.rows <= MGS_NR * S && threads <= 1024) {
          put(reg[threads <= 512 ? 1 : 0], p, 0);
          continue;
       }
-      constexpr int rows_a_lane[4] = {96, 64, 48, 32};
-      int c = d.rows <= 32 * S ? 3 : (d.rows <= 48 * S ? 2 : (d.rows <= 64 * S ? 1 : 0));
-      if (d.rows <= MGS_NR * S) c = S == 64 ? 4 : (S == 32 ? 5 : (S == 16 ? 6 : (S == 8 ? 7 : 8)));
-      const int nrs = (c < 4 ? rows_a_lane[c] : MGS_NR) * S;
+      d.shape = MGS_96x64;
+      int rows_a_lane = 96;
+      if (d.rows <= MGS_NR * S) {
+         d.shape = S == 64 ? MGS_16x64 : (S == 32 ? MGS_16x32 : (S == 16 ? MGS_16x16 : (S == 8 ? MGS_16x8 : MGS_16x4)));
+         rows_a_lane = MGS_NR;
+      } else if (d.rows <= 64 * S) {
+         d.shape = d.rows <= 32 * S ? MGS_32x64 : (d.rows <= 48 * S ? MGS_48x64 : MGS_64x64);
+         rows_a_lane = d.rows <= 32 * S ? 32 : (d.rows <= 48 * S ? 48 : 64);
+      }
+      const int nrs = rows_a_lane * S;
       d.nb = 4;
       while (d.nb > 1 && mgs_blk_bytes(nrs, d.cols, d.nb) > LDS_MAX) d.nb >>= 1;
       // (the kernel's offsets into a matrix are 32 bits)
       if (S > 1 && d.rows <= nrs && mgs_blk_bytes(nrs, d.cols, d.nb) <= LDS_MAX) {
-         put(blk[c], p, mgs_blk_bytes(nrs, d.cols, d.nb));
+         put(blk[rows_a_lane <= 48 ? 1 : 0], p, mgs_blk_bytes(nrs, d.cols, d.nb));
          continue;
       }
       d.ws_off = (long long)ws;
       ws += mgs_long_bytes(d.cols);
       put(large, p, 0);
    }
+   // Launches of one stream run one after the other: those that would not fill
+   // the chip join the next larger ones, with a lane per column by threads first
+   // (at most as many as the kernel takes), then by rows.
+   if (reg[1].list.size() < 512 && !reg[0].list.empty()) {
+      for (int p : reg[1].list) put(reg[0], p, 0);
+      reg[1].list.clear();
+   }
+   for (int n = 0; n < 3; n++)
+      for (int c = 0; c < 4; c++)
+         if (!cols[n][c].list.empty() && cols[n][c].list.size() < 512 && (128 << c) <= mgs_cols_threads(cols_rows[n])) {
+            bool larger = false;
+            for (int k = c + 1; k < 5; k++) larger = larger || !cols[n][k].list.empty();
+            if (!larger) break;
+            for (int p : cols[n][c].list) put(cols[n][c + 1], p, cols_lds(p, n));
+            cols[n][c].list.clear();
+         }
+   for (int n = 0; n < 2; n++)
+      for (int c = 0; c < 5; c++)
+         if (cols[n][c].list.size() < 512 && (64 << c) <= mgs_cols_threads(cols_rows[n + 1]) &&
+             !cols[n + 1][c].list.empty()) {
+            for (int p : cols[n][c].list) put(cols[n + 1][c], p, cols_lds(p, n + 1));
+            cols[n][c].list.clear();
+         }
    // the largest ahead: they run longest
    auto longest_first = [&](Class& c) {
       std::stable_sort(c.list.begin(), c.list.end(), [&](int x, int y) {
@@ -830,19 +886,14 @@ void run_mgs(std::vector<MgsDesc>& descs, double* A, double* Q, std::vector<int>
    dl.upload(all, s);
    dr.alloc(nprob);
    if (ws) dws.alloc(ws);
-   auto k96 = k_mgs_blk<96, 64, 512, false>, k64 = k_mgs_blk<64, 64, 512, false>;
-   auto k48 = k_mgs_blk<48, 64, 768, false>, k32 = k_mgs_blk<32, 64, 1024, false>;
-   decltype(k96) k16[5] = {k_mgs_blk<16, 64, 1024, true>, k_mgs_blk<16, 32, 1024, true>, k_mgs_blk<16, 16, 1024, true>,
-                           k_mgs_blk<16, 8, 1024, true>, k_mgs_blk<16, 4, 1024, true>};
    static std::once_flag attr;
-   std::call_once(attr, [&] {
-      for (const void* k : {(const void*)k96, (const void*)k64, (const void*)k48, (const void*)k32,
-                            (const void*)k16[0], (const void*)k16[1], (const void*)k16[2], (const void*)k16[3],
-                            (const void*)k16[4], (const void*)k_mgs_cols<32>, (const void*)k_mgs_cols<64>,
-                            (const void*)k_mgs_cols<96>})
+   std::call_once(attr, [] {
+      for (const void* k : {(const void*)k_mgs_blk<512>, (const void*)k_mgs_blk<768>, (const void*)k_mgs_cols<32>,
+                            (const void*)k_mgs_cols<64>, (const void*)k_mgs_cols<96>})
          FSVD_CHECK(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)LDS_MAX));
    });
    const int* l = dl.p;
+   int launches = 0;
    if (!large.list.empty())
       hipLaunchKernelGGL(k_mgs_long, dim3((unsigned)large.list.size()), dim3(MGS_LT), 0, s, dd.p, l, A, Q, dr.p, eps,
                          dws.p);
@@ -851,12 +902,10 @@ void run_mgs(std::vector<MgsDesc>& descs, double* A, double* Q, std::vector<int>
       const unsigned n = (unsigned)c.list.size();
       if (n) hipLaunchKernelGGL(kernel, dim3(n), dim3(threads), c.lds, s, dd.p, l, A, Q, dr.p, eps);
       l += n;
+      launches += n > 0;
    };
-   launch(k96, blk[0], 512);
-   launch(k64, blk[1], 512);
-   launch(k48, blk[2], 768);
-   launch(k32, blk[3], 1024);
-   for (int c = 0; c < 5; c++) launch(k16[c], blk[4 + c], 1024);
+   launch(k_mgs_blk<512>, blk[0], 512);
+   launch(k_mgs_blk<768>, blk[1], 768);
    launch(k_mgs_reg<1024>, reg[0], 1024);
    launch(k_mgs_reg<512>, reg[1], 512);
    for (int c = 0; c < 5; c++) launch(k_mgs_cols<32>, cols[0][c], 64 << c);
@@ -867,12 +916,10 @@ void run_mgs(std::vector<MgsDesc>& descs, double* A, double* Q, std::vector<int>
    FSVD_CHECK(hipMemcpyAsync(h.data(), dr.p, sizeof(int) * nprob, hipMemcpyDeviceToHost, s));
    FSVD_CHECK(hipStreamSynchronize(s));
    for (int i = 0; i < nprob; i++) ranks[descs[i].rank_slot] = h[descs[i].rank_slot];
-   if (const char* e = std::getenv("FFTSVD_TIMING"); e && e[0] == '1') {
-      std::fprintf(stderr, "[fftsvd mgs] %d problems: %zu large, blocked", nprob, large.list.size());
-      for (const Class& c : blk) std::fprintf(stderr, " %zu", c.list.size());
-      std::fprintf(stderr, ", in registers %zu %zu, the others a lane per column\n", reg[0].list.size(),
-                   reg[1].list.size());
-   }
+   if (const char* e = std::getenv("FFTSVD_TIMING"); e && e[0] == '1')
+      std::fprintf(stderr, "[fftsvd mgs] %d problems: %zu large, %zu + %zu blocked, %zu in registers, the others a "
+                   "lane per column; %d launches\n", nprob, large.list.size(), blk[0].list.size(), blk[1].list.size(),
+                   reg[0].list.size() + reg[1].list.size(), launches);
 }
 
 void launch_f64_to_f32(const double* a, float* b, long long n, hipStream_t s) {
