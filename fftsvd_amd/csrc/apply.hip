@@ -2122,13 +2122,15 @@ __global__ void __launch_bounds__(256) k_leaf_mc(const LeafDesc* __restrict__ le
 // shared between blocks (one scatter per block with FP64 atomics took 87 us a
 // tree at 31 000 panels, beside ~60 per-level launches for the far field).
 // Bound by latency: short gathers (32 rows per neighbour block, 20-60 columns),
-// 39 us a launch at 31 000 panels with 7 waves per SIMD.  Transposed product of
-// both trees, host to host: 31 000 panels 1.22 to 0.28 ms FP32, 1.49 to 0.39
-// FP64; 100 000 panels 2.38 to 0.67 and 2.89 to 1.03.  Near field: the rows of all blocks are listed in
-// LDS (TILE at a time: entry offset, column stride, x), lanes take rows, waves
-// four columns each with both layers of a column in flight; FP64 sums.  Far
-// field: 16 lanes per panel over the rows of its panel-major basis, summed in
-// T per source cube and in FP64 over the cubes.
+// 39 us a launch at 31 000 panels with 7 waves per SIMD.  It moves 279 MB (FP32)
+// and 548 MB (FP64) a tree at 100 000 panels, the forward k_leaf 254 and 501.
+// Transposed product of both trees, host to host: 31 000 panels 1.22 to 0.27 ms
+// FP32, 1.49 to 0.38 FP64; 100 000 panels 2.38 to 0.63 and 2.89 to 1.00.  Near
+// field: the rows of all blocks are listed in LDS (TILE at a time: entry offset,
+// column stride, x), lanes take rows, waves four columns each with both layers
+// of a column in flight; FP64 sums.  Far field: 16 lanes per panel over the rows
+// of its panel-major basis, summed in T per source cube and in FP64 over the
+// cubes.
 constexpr int LT_TILE = 512;
 template <typename T>
 __global__ void __launch_bounds__(256, sizeof(T) == 4 ? 7 : 5) k_leaf_t(const LeafT* __restrict__ leaves, const NearT* __restrict__ nbr,

@@ -1,8 +1,9 @@
-"""Sampled column and row bases (pivoted MGS) over the sizes that the two
-kernels take: ranks equal to the oracle's for leaf sizes and SVD tolerances
-that fill the register kernel's launches, the blocked kernel in LDS, and its
-form in global scratch (cubes of 20480 panels); bases orthonormal to the
-level that pivoted MGS keeps, eps / svdeps times a factor for the sums."""
+"""Sampled column and row bases (pivoted MGS) over the sizes that their kernels
+take: ranks equal to the oracle's for leaf sizes and SVD tolerances that reach a
+lane per column (rows in registers, and beyond them in LDS), two columns a lane
+group, the blocked kernel, and the one for the longest columns (cubes of 20480
+panels); bases orthonormal to the level that pivoted MGS keeps, eps / svdeps
+times a factor for the sums.  Their rounding: tests/test_gpu_fp64_products.py."""
 import numpy as np
 import pytest
 
