@@ -36,9 +36,11 @@ class DeviceCache {
    void* take(size_t bytes) {
       const int dev = Api::device();
       const size_t want = rounded(bytes);
+      bool bounded = false;
       {
          std::lock_guard<std::mutex> g(mu_);
          Device& d = devices_[dev];
+         bounded = d.limit > 0;
          // the smallest kept block that wastes at most a quarter of the request
          auto it = d.kept.lower_bound(want);
          if (it != d.kept.end() && it->first <= want + want / 4) {
@@ -57,10 +59,10 @@ class DeviceCache {
          p = Api::alloc(want);
          if (!p) return nullptr;
       }
-      const size_t total = Api::total();
+      const size_t total = bounded ? 0 : Api::total();
       std::lock_guard<std::mutex> g(mu_);
       live_[p] = {want, dev};
-      devices_[dev].limit = total ? total / 24 : (size_t)1 << 30;
+      if (!bounded) devices_[dev].limit = total ? total / 24 : (size_t)1 << 30;
       return p;
    }
 

@@ -761,7 +761,8 @@ namespace fsvd {
 void launch_integral_blocks(int nblk, const IntBlock* blocks, const double* bpts, const int* bpan,
                             const PanelGeom* panels, int kernel, double kappa, double* out, hipStream_t s) {
    if (nblk > 0)
-      hipLaunchKernelGGL(k_integral_blocks, dim3(nblk), dim3(256), 0, s, blocks, bpts, bpan, panels, kernel, kappa, out);
+      hipLaunchKernelGGL(k_integral_blocks, dim3(nblk), dim3(256), 0, s, blocks, bpts, bpan, panels, kernel, kappa,
+                         out);
 }
 
 void launch_green_blocks(int nblk, const GreenBlock* blocks, const double* dest, const double* src, int kernel,
